@@ -336,6 +336,20 @@ __global__ void k_add_extra(VertexDev V, const int64_t* ids, const double* force
   V.f[2 * V.vs + i] += forces[3 * k + 2];
 }
 
+// Vertex read-back: plane sets interleaved by vertex, written straight into pinned
+// host memory (bound by the link, 56 GB/s; a wavefront stores one run of 512
+// bytes, the plane reads of neighbouring wavefronts share cache lines).
+struct PlaneSets {
+  const double* p[3];
+};
+__global__ __launch_bounds__(BLOCK) void k_interleave(PlaneSets S, int64_t vs, int64_t k0, uint32_t n3,
+                                                      double* __restrict__ out) {
+  const uint32_t e = blockIdx.x * BLOCK + threadIdx.x;
+  if (e >= n3) return;
+  const uint32_t k = e / 3, c = e - 3 * k;
+  out[(int64_t)blockIdx.y * n3 + e] = S.p[blockIdx.y][c * vs + k0 + k];
+}
+
 inline dim3 grid_for(int64_t n) { return dim3((unsigned)((n + BLOCK - 1) / BLOCK)); }
 
 }  // namespace
@@ -398,6 +412,17 @@ hipError_t launch_interp_advance(hipStream_t s, const VertexDev& V, const R* uf,
 hipError_t launch_add_extra_force(hipStream_t s, const VertexDev& V, const int64_t* ids, const double* forces, int n) {
   if (n <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_add_extra, grid_for(n), dim3(BLOCK), 0, s, V, ids, forces, n);
+  return hipGetLastError();
+}
+
+hipError_t launch_interleave(hipStream_t s, const double* const* src, int nf, int64_t vs, int64_t k0, int64_t n,
+                             double* out) {
+  if (n <= 0 || nf <= 0) return hipSuccess;
+  if (nf > 3 || 3 * n > UINT32_MAX - BLOCK) return hipErrorInvalidValue;
+  PlaneSets S{};
+  for (int k = 0; k < nf; ++k) S.p[k] = src[k];
+  const dim3 g = grid_for(3 * n);
+  hipLaunchKernelGGL(k_interleave, dim3(g.x, (unsigned)nf), dim3(BLOCK), 0, s, S, vs, k0, (uint32_t)(3 * n), out);
   return hipGetLastError();
 }
 

@@ -24,12 +24,13 @@ template <typename R>
 hipError_t launch_init_equilibrium(hipStream_t s, R* f, const uint8_t* type, const LatticeDev& L,
                                    double rho, const double u[3]);
 template <typename R>
-hipError_t launch_natural_populations(hipStream_t s, const R* f, double* out, const LatticeDev& L, int phase);
+hipError_t launch_natural_populations(hipStream_t s, const R* f, double* out, const LatticeDev& L, int phase,
+                                      int64_t n0, int64_t n);  // nodes n0..n0+n-1: out[i * n + node - n0]
 template <typename R>
 hipError_t launch_store_populations(hipStream_t s, R* f, const double* in, const LatticeDev& L);
 template <typename R>
 hipError_t launch_fluid_moments(hipStream_t s, const R* f, const R* Fcur, const uint8_t* type, const LatticeDev& L,
-                                int phase, const CollideArgs& a, double* rho, double* u);
+                                int phase, const CollideArgs& a, int64_t n0, int64_t n, double* rho, double* u);
 // per-block {min, max, sum, count} of |u| (what 0) or |Fstat| (what 1) over the
 // non-bounce-back nodes; nblocks * 4 doubles in partials
 template <typename R>
@@ -70,6 +71,10 @@ template <typename R>
 hipError_t launch_interp_advance(hipStream_t s, const VertexDev& V, const R* uf, const uint8_t* type,
                                  const LatticeDev& L, int do_interp, int do_advance, unsigned long long* wall_hits);
 hipError_t launch_add_extra_force(hipStream_t s, const VertexDev& V, const int64_t* ids, const double* forces, int n);
+// nf <= 3 sets of 3 planes (stride vs), vertices k0..k0+n-1, interleaved by vertex:
+// out[k * 3 n + 3 (vertex - k0) + c]
+hipError_t launch_interleave(hipStream_t s, const double* const* src, int nf, int64_t vs, int64_t k0, int64_t n,
+                             double* out);
 
 // fused per-cell step (hc_cell_body.h): interpolation + advance, mechanics, next spread
 enum { CELL_FLAG_INTERP = 1, CELL_FLAG_MECH = 2, CELL_FLAG_SPREAD = 4, CELL_FLAG_REPULSION = 8 };

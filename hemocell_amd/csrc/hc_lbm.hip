@@ -312,13 +312,15 @@ __device__ __forceinline__ R post_stream(const R* f, const LatticeDev& L, int ph
   return f[opp(i) * L.stride + (int64_t)Z + (int64_t)L.nz * ((int64_t)Y + (int64_t)L.ny * X)];
 }
 
+// nodes n0..n0+cnt-1; out (pinned host memory): plane i at out + i * cnt
 template <typename R>
-__global__ void k_natural(const R* f, double* out, LatticeDev L, int phase) {
-  const int64_t n = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-  if (n >= L.N) return;
+__global__ __launch_bounds__(BLOCK) void k_natural(const R* f, double* out, LatticeDev L, int phase, int64_t n0,
+                                                   int64_t cnt) {
+  const int64_t k = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+  if (k >= cnt) return;
   int x, y, z;
-  coords(n, L, x, y, z);
-  for (int i = 0; i < 19; ++i) out[i * L.N + n] = (double)post_stream(f, L, phase, x, y, z, i, n);
+  coords(n0 + k, L, x, y, z);
+  for (int i = 0; i < 19; ++i) out[i * cnt + k] = (double)post_stream(f, L, phase, x, y, z, i, n0 + k);
 }
 
 template <typename R>
@@ -364,19 +366,28 @@ __device__ void node_moments(const R* f, const R* Fcur, const uint8_t* type, con
   rho = rb + 1.0;
 }
 
+// Density and velocity of the nodes n0..n0+cnt-1 into rho and u, which lie in
+// pinned host memory: bound by the link (56 GB/s).  The interleaved velocities
+// go through LDS so that every store of a wavefront is one run of 512 bytes.
 template <typename R>
-__global__ void k_moments(const R* f, const R* Fcur, const uint8_t* type, LatticeDev L, int phase, CollideArgs a,
-                          double* rho, double* u) {
-  const int64_t n = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-  if (n >= L.N) return;
-  double r, u0, u1, u2;
-  node_moments<R>(f, Fcur, type, L, phase, a, n, r, u0, u1, u2);
-  if (rho) rho[n] = r;
-  if (u) {
-    u[3 * n + 0] = u0;
-    u[3 * n + 1] = u1;
-    u[3 * n + 2] = u2;
+__global__ __launch_bounds__(BLOCK) void k_moments(const R* f, const R* Fcur, const uint8_t* type, LatticeDev L,
+                                                   int phase, CollideArgs a, int64_t n0, int64_t cnt, double* rho,
+                                                   double* u) {
+  __shared__ double su[3 * BLOCK];
+  const int64_t first = (int64_t)blockIdx.x * BLOCK;
+  const int64_t k = first + threadIdx.x;
+  if (k < cnt) {
+    double r, u0, u1, u2;
+    node_moments<R>(f, Fcur, type, L, phase, a, n0 + k, r, u0, u1, u2);
+    if (rho) rho[k] = r;
+    su[3 * threadIdx.x + 0] = u0;
+    su[3 * threadIdx.x + 1] = u1;
+    su[3 * threadIdx.x + 2] = u2;
   }
+  __syncthreads();
+  if (!u) return;
+  const int n = 3 * (int)(cnt - first < BLOCK ? cnt - first : BLOCK);
+  for (int e = threadIdx.x; e < n; e += BLOCK) u[3 * first + e] = su[e];
 }
 
 // FluidInfo statistics (helper/fluidInfo.cpp:27-102): minimum, maximum and sum of
@@ -591,8 +602,10 @@ hipError_t launch_init_equilibrium(hipStream_t s, R* f, const uint8_t* type, con
 }
 
 template <typename R>
-hipError_t launch_natural_populations(hipStream_t s, const R* f, double* out, const LatticeDev& L, int phase) {
-  hipLaunchKernelGGL((k_natural<R>), grid_for(L.N), dim3(BLOCK), 0, s, f, out, L, phase);
+hipError_t launch_natural_populations(hipStream_t s, const R* f, double* out, const LatticeDev& L, int phase,
+                                      int64_t n0, int64_t n) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL((k_natural<R>), grid_for(n), dim3(BLOCK), 0, s, f, out, L, phase, n0, n);
   return hipGetLastError();
 }
 
@@ -604,8 +617,9 @@ hipError_t launch_store_populations(hipStream_t s, R* f, const double* in, const
 
 template <typename R>
 hipError_t launch_fluid_moments(hipStream_t s, const R* f, const R* Fcur, const uint8_t* type, const LatticeDev& L,
-                                int phase, const CollideArgs& a, double* rho, double* u) {
-  hipLaunchKernelGGL((k_moments<R>), grid_for(L.N), dim3(BLOCK), 0, s, f, Fcur, type, L, phase, a, rho, u);
+                                int phase, const CollideArgs& a, int64_t n0, int64_t n, double* rho, double* u) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL((k_moments<R>), grid_for(n), dim3(BLOCK), 0, s, f, Fcur, type, L, phase, a, n0, n, rho, u);
   return hipGetLastError();
 }
 
@@ -664,10 +678,10 @@ hipError_t launch_lees_edwards(hipStream_t s, R* f, const uint8_t* type, const L
                                                const CollideArgs&, int, bool, const uint32_t*, int, bool);    \
   template hipError_t launch_init_equilibrium<R>(hipStream_t, R*, const uint8_t*, const LatticeDev&, double,    \
                                                  const double*);                                              \
-  template hipError_t launch_natural_populations<R>(hipStream_t, const R*, double*, const LatticeDev&, int);    \
+  template hipError_t launch_natural_populations<R>(hipStream_t, const R*, double*, const LatticeDev&, int, int64_t, int64_t); \
   template hipError_t launch_store_populations<R>(hipStream_t, R*, const double*, const LatticeDev&);           \
   template hipError_t launch_fluid_moments<R>(hipStream_t, const R*, const R*, const uint8_t*, const LatticeDev&,  \
-                                              int, const CollideArgs&, double*, double*);                     \
+                                              int, const CollideArgs&, int64_t, int64_t, double*, double*);   \
   template hipError_t launch_fluid_stats<R>(hipStream_t, const R*, const R*, const uint8_t*, const LatticeDev&,    \
                                             int, const CollideArgs&, const R*, int, double*, int);             \
   template hipError_t launch_fill_zero<R>(hipStream_t, R*, int64_t);                                            \
