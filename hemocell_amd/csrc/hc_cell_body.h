@@ -394,12 +394,9 @@ __device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev
         V.f[2 * vs + i] = f2;
       }
     }
-    for (int a = 0; a < 3; ++a) {
-      atomicMin(&bmin[a], lmin[a]);
-      atomicMax(&bmax[a], lmax[a]);
-    }
-    if (lbad) atomicOr(&bad, 1);
-    if (lfar) atomicOr(&farpk, 1);
+    block_bounds(lmin, lmax, bmin, bmax);
+    if (lbad) bad = 1;
+    if (lfar) farpk = 1;
     // the spread box starts at zero (each slab's flush clears what it used), and
     // so do the plane counts of the bucketing
     for (int e = tid; e < 3 * box_nodes; e += BS) box[e] = 0.0;

@@ -266,11 +266,8 @@ __global__ __launch_bounds__(BS) void k_spread_cells(VertexDev V, R* __restrict_
       lmax[a] = max(lmax[a], c);
     }
   }
-  for (int a = 0; a < 3; ++a) {
-    atomicMin(&bmin[a], lmin[a]);
-    atomicMax(&bmax[a], lmax[a]);
-  }
-  if (lbad) atomicOr(&bad, 1);
+  block_bounds(lmin, lmax, bmin, bmax);
+  if (lbad) bad = 1;
   __syncthreads();
   // support nodes of a vertex are floor(p) and floor(p) + 1 on each axis
   const int o0 = bmin[0], o1 = bmin[1], o2 = bmin[2];
