@@ -645,6 +645,30 @@ hc_status do_visc_membrane(hc_ctx* ctx, const double* xold) {
   return HC_OK;
 }
 
+// Spread scratch in LDS of one cell (bytes, beside the 2 bytes per vertex of the
+// layout's list): a row mask of 12 bytes per (x, y) row of the support box and 28
+// per support node in one pass.  An RBC touches ~1290 nodes in at most 306 rows, a
+// platelet at most 97 in 36, the 8 um WBC 2210 in 324.
+// Many cells: an RBC's spread takes two passes, so that five FP32 (four FP64)
+// workgroups share a compute unit's 160 KB: 15.5k RBC, FP32 step 3.12 ms with
+// 18432 bytes (three passes), 3.08 with 21504, 3.31 with 24576 (four workgroups),
+// 3.48 with 40960 (one pass, three workgroups).
+// Few cells, which occupy a compute unit alone: everything in one pass.
+int spread_box_bytes(const hc_ctx* c, int model, bool few) {
+  if (c->spread_lds > 0) return c->spread_lds;
+  if (model == HC_MODEL_PLT) return 6144;
+  if (!few) return 21504;
+  return model == HC_MODEL_WBC ? 69632 : 45056;
+}
+
+// Threads of one cell's workgroup.  Fewer cells than compute units: their latency,
+// not the occupancy, sets the time, and the widest block wins (a platelet's 66
+// vertices: four wavefronts, which shorten its box clear and flush).
+int cell_threads(const hc_ctx* c, int model, bool few) {
+  if (few && !(c->cell_block_env && model == HC_MODEL_RBC)) return 1024;
+  return model == HC_MODEL_WBC ? c->wbc_block : (model == HC_MODEL_PLT ? 64 : c->cell_block);
+}
+
 // every type in one persistent launch on the context stream; false when the
 // launch does not apply (no queue, or the layout does not fit the LDS)
 template <typename R>
@@ -662,7 +686,7 @@ bool mixed_cell_step(hc_ctx* ctx, int do_interp, hc_status& st) {
     if (ctx->repulsion) f |= CELL_FLAG_REPULSION;
     flags[t] = f;
   }
-  const int box = ctx->spread_lds > 0 ? ctx->spread_lds : 12288;
+  const int box = spread_box_bytes(ctx, HC_MODEL_RBC, false);
   const hipError_t e = launch_cell_step_mixed<R>(
       ctx->stream, vdev(ctx), ctx->d_types, ht.data(), (int)ht.size(), flags.data(), ctx->d_queue, ctx->nqueue,
       ctx->d_head, ctx->mixed_per_cu * ctx->n_cu, ctx->d_cell_base, (const R*)ctx->ufield, ctx->type, ctx->L,
@@ -708,12 +732,14 @@ hc_status do_cell_step(hc_ctx* ctx, int do_interp) {
     if (do_interp) flags |= CELL_FLAG_INTERP;
     if ((ctx->iter % tb.host.timescale) == 0) flags |= CELL_FLAG_MECH;
     if (ctx->repulsion) flags |= CELL_FLAG_REPULSION;
-    // spread box in LDS; larger supports are spread in slabs of x-planes
-    const int box = ctx->spread_lds > 0 ? ctx->spread_lds : 12288;
-    // few cells: their latency, not the occupancy, sets the time: the widest block
-    int block = tb.host.model == HC_MODEL_WBC ? ctx->wbc_block : ctx->cell_block;
-    if (tb.ncells < ctx->n_cu && !(ctx->cell_block_env && tb.host.model == HC_MODEL_RBC)) block = 1024;
-    const bool gpos = k != 0 && nside > 0 && ctx->side_gpos && 3 * (size_t)tb.host.nv * sizeof(double) > 32768;
+    const bool few = tb.ncells < ctx->n_cu;
+    int block = cell_threads(ctx, tb.host.model, few);
+    // while compute units are left over beside the main type, a large side cell
+    // takes one for itself with its positions in LDS: one 2562-vertex WBC beside
+    // 242 RBC, 350 -> 121 us per step
+    const bool gpos = k != 0 && nside > 0 && ctx->side_gpos && 3 * (size_t)tb.host.nv * sizeof(double) > 32768 &&
+                      act[0]->ncells + tb.ncells > ctx->n_cu;
+    const int box = spread_box_bytes(ctx, tb.host.model, few && !gpos);
     if (gpos) block = 256;
     HC_TRY(launch_cell_step<R>(st, vdev(ctx), tb.dev, tb.d_cells, tb.ncells, ctx->d_cell_base, (const R*)ctx->ufield,
                                ctx->type, ctx->L, (R*)ctx->Fibm[1 - ctx->cur], ctx->d_extra_dense, ctx->bend,
@@ -1177,7 +1203,6 @@ hc_status batch_impl(hc_ctx* const* cs, int n, int nsteps) {
   HC_TRY(hipMemcpyAsync(lead->d_batch[slot], lead->h_batch[slot], bytes.size(), hipMemcpyHostToDevice, lead->stream),
          "hipMemcpyAsync");
   const unsigned char* base = (const unsigned char*)lead->d_batch[slot];
-  const int box = lead->spread_lds > 0 ? lead->spread_lds : 12288;
   for (int k = 0; k < nsteps; ++k) {
     for (const Group& g : groups[k & 1]) {
       if (g.kind == 0) {
@@ -1204,12 +1229,9 @@ hc_status batch_impl(hc_ctx* const* cs, int n, int nsteps) {
       if (g.kind == 2) {
         hipStream_t st = (gi == 0 || nside == 0) ? lead->stream : lead->side[(gi - 1) % nside];
         ++gi;
-        // the lead context's launch shapes, chosen as do_cell_step chooses them:
-        // fewer cells than compute units take the widest block (platelets: 256
-        // threads instead of 64), unless HC_CELL_BLOCK fixes the RBC block
-        int block = g.T.model == HC_MODEL_WBC ? lead->wbc_block
-                                              : (g.T.model == HC_MODEL_PLT ? 64 : lead->cell_block);
-        if (g.count < lead->n_cu && !(lead->cell_block_env && g.T.model == HC_MODEL_RBC)) block = 1024;
+        // the lead context's launch shapes, chosen as do_cell_step chooses them
+        const bool few = g.count < lead->n_cu;
+        const int block = cell_threads(lead, g.T.model, few), box = spread_box_bytes(lead, g.T.model, few);
         HC_TRY(launch_cell_step_multi<R>(st, g.T, (const CellCase*)(base + g.offset), g.count, box, lead->lds_device,
                                          block),
                "batched cell_step");

@@ -9,9 +9,9 @@
 //      ParticleMechanics) on the positions in LDS;
 //   3. spreadParticleForce of step t+1 (:841-863): the forces just computed (plus
 //      any extra force, capped to f_limit in place) are spread from the same
-//      positions into the force buffer of the next step, through an LDS box
-//      covering the cell's support and one global atomic per non-zero node.
-//      The box holds doubles in both precisions: LDS double atomic adds run
+//      positions into the force buffer of the next step, through one sum in LDS
+//      per support node of the cell and one global atomic per non-zero sum.
+//      The sums are doubles in both precisions: LDS double atomic adds run
 //      several times faster than float ones on this chip.
 // Step t+1's spread needs exactly x_t and F(x_t), which steps 1-2 produce, so
 // doing it here saves reloading the cell.  Positions stay in LDS for the whole
@@ -32,8 +32,6 @@ namespace hcg {
 namespace {
 
 enum { CELL_INTERP = 1, CELL_MECH = 2, CELL_SPREAD = 4, CELL_REPULSION = 8 };
-// x-planes of a cell's support box up to which the spread buckets its vertices
-constexpr int kMaxPlanes = 64;
 // 64-triangle chunks of a mesh whose volume is summed in an order independent of
 // the block size (meshes up to 8192 triangles)
 constexpr int kVolChunks = 128;
@@ -66,7 +64,7 @@ __device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev
   __shared__ double red[kVolChunks];
   __shared__ double vforce_sh;
   __shared__ int bmin[3], bmax[3], bad, farpk;
-  __shared__ int pcount[kMaxPlanes + 1], pstart[kMaxPlanes + 1];
+  __shared__ int wsum[BS / 64];
   const int tid = threadIdx.x;
   const int nv = T.nv;
   const int64_t vs = V.vs;
@@ -137,13 +135,41 @@ __device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev
   auto pos_z = [&](int k) -> double {
     return REL ? (use_pk ? unpack(fo2, pk[2 * nv + k]) : V.x[2 * vs + base + k]) : (double)pz[k];
   };
-  double* box = region;
-  // after the box: the spread's vertex list, bucketed by x-plane
-  uint16_t* vlist = reinterpret_cast<uint16_t*>(region + 3 * (int64_t)box_nodes);
+  // low corner and support of vertex k for the spread; from a packed position
+  // without double arithmetic
+  const int foi[3] = {(int)fo0, (int)fo1, (int)fo2};
+  auto low_node = [&](int k, int (&n0)[3]) {
+    if (REL && use_pk) {
+#pragma unroll
+      for (int a = 0; a < 3; ++a) n0[a] = foi[a] + (int)(pk[a * nv + k] >> 24) - 128;
+    } else {
+      n0[0] = (int)floor(pos_x(k));
+      n0[1] = (int)floor(pos_y(k));
+      n0[2] = (int)floor(pos_z(k));
+    }
+  };
+  auto support_of = [&](int k, SupportT<SW>& sp) {
+    if (REL && use_pk) {
+      int n0[3];
+      SW q[3][2];
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const uint32_t w = pk[a * nv + k];
+        n0[a] = foi[a] + (int)(w >> 24) - 128;
+        q[a][1] = (SW)(w & 0xFFFFFFu) * SW(1.0 / 16777216.0);
+        q[a][0] = SW(1) - q[a][1];
+      }
+      finish_support(n0, q, true, [&](int a) { return (double)n0[a]; }, L, type, sp);
+    } else {
+      ibm_support(pos_x(k), pos_y(k), pos_z(k), L, type, sp);
+    }
+  };
+  // the spread's scratch: the region and the list bytes after it
+  const int scratch_bytes = 24 * box_nodes + (int)cell_list_bytes(nv);
 
   // ---- 1. interpolation and advance ------------------------------------------
-  // A thread takes up to U of its vertices at once, so their position loads and
-  // support-node gathers are in flight together.
+  // A thread takes up to U of its vertices at once, so their position loads are in
+  // flight together.
   // A vertex removed by wall contact (flag) stays where it is and spreads
   // nothing; its cell is incomplete from then on (hemoCellParticleField.cpp:
   // 566-588 removes it; applyConstitutiveModel, :633-675, skips cells with a
@@ -151,7 +177,7 @@ __device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev
   constexpr int U = 3;
   bool lrem = false;
   for (int k0 = tid; k0 < nv; k0 += U * BS) {
-    double xa[U][3], va[U][3];
+    double xa[U][3];
     bool gone[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -178,37 +204,40 @@ __device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev
         if (STAGED && visc) vx[k] = vy[k] = vz[k] = P(0);
         continue;
       }
+      double v0, v1, v2;
       if (flags & CELL_INTERP) {
         SupportT<SW> sp;
         ibm_support(xa[u][0], xa[u][1], xa[u][2], L, type, sp);
-        SW v0 = SW(0), v1 = SW(0), v2 = SW(0);
+        // four nodes at a time, the ones without weight too, so that their reads are
+        // in flight together (behind a test per node each was waited for alone;
+        // eight at a time take the registers of a wavefront per SIMD)
+        SW w0 = SW(0), w1 = SW(0), w2 = SW(0);
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          if (sp.w[q] == SW(0)) continue;
-          const R* un = uf + 3 * (int64_t)sp.idx[q];
-          v0 += (SW)un[0] * sp.w[q];
-          v1 += (SW)un[1] * sp.w[q];
-          v2 += (SW)un[2] * sp.w[q];
+        for (int h = 0; h < 8; h += 4) {
+          R un[4][3];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const R* at = uf + 3 * (uint64_t)sp.idx[h + q];
+            un[q][0] = at[0];
+            un[q][1] = at[1];
+            un[q][2] = at[2];
+          }
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const bool on = sp.w[h + q] != SW(0);
+            w0 += (on ? (SW)un[q][0] : SW(0)) * sp.w[h + q];
+            w1 += (on ? (SW)un[q][1] : SW(0)) * sp.w[h + q];
+            w2 += (on ? (SW)un[q][2] : SW(0)) * sp.w[h + q];
+          }
+          __builtin_amdgcn_sched_barrier(0);
         }
-        va[u][0] = (double)v0;
-        va[u][1] = (double)v1;
-        va[u][2] = (double)v2;
+        V.v[i] = v0 = (double)w0;
+        V.v[vs + i] = v1 = (double)w1;
+        V.v[2 * vs + i] = v2 = (double)w2;
       } else {
-        va[u][0] = V.v[i];
-        va[u][1] = V.v[vs + i];
-        va[u][2] = V.v[2 * vs + i];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = k0 + u * BS;
-      if (k >= nv || gone[u]) continue;
-      const int64_t i = base + k;
-      const double v0 = va[u][0], v1 = va[u][1], v2 = va[u][2];
-      if (flags & CELL_INTERP) {
-        V.v[i] = v0;
-        V.v[vs + i] = v1;
-        V.v[2 * vs + i] = v2;
+        v0 = V.v[i];
+        v1 = V.v[vs + i];
+        v2 = V.v[2 * vs + i];
       }
       const double x0 = xa[u][0] + v0, x1 = xa[u][1] + v1, x2 = xa[u][2] + v2;
       if (REL && k == 0) {
@@ -234,15 +263,17 @@ __device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev
       if (type && isfinite(x0) && isfinite(x1) && isfinite(x2)) {
         const double p[3] = {x0, x1, x2};
         const int dims[3] = {L.nx, L.ny, L.nz};
-        int64_t wc[3];
+        int wc[3];
         bool out = false;
+#pragma unroll
         for (int a = 0; a < 3; ++a) {
-          const int64_t cc = (int64_t)floor(p[a] + 0.5);
-          if (cc >= 0 && cc < dims[a]) wc[a] = cc;
-          else if (L.periodic[a]) wc[a] = wrap_mod(cc, dims[a]);
+          const double fl = floor(p[a] + 0.5);
+          if (fl >= 0.0 && fl < (double)dims[a]) wc[a] = (int)fl;
+          else if (L.periodic[a]) wc[a] = wrap_node(fl, dims[a]);
           else out = true;
         }
-        if (!out && type[wc[2] + (int64_t)L.nz * (wc[1] + (int64_t)L.ny * wc[0])] != HC_NODE_FLUID) {
+        if (!out && type[(uint32_t)wc[2] + (uint32_t)L.nz * ((uint32_t)wc[1] + (uint32_t)L.ny * (uint32_t)wc[0])] !=
+                        HC_NODE_FLUID) {
           atomicAdd(wall_hits, 1ull);
           if (V.flag) V.flag[i] = VFLAG_REMOVED;
           lrem = true;
@@ -397,19 +428,26 @@ __device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev
     block_bounds(lmin, lmax, bmin, bmax);
     if (lbad) bad = 1;
     if (lfar) farpk = 1;
-    // the spread box starts at zero (each slab's flush clears what it used), and
-    // so do the plane counts of the bucketing
-    for (int e = tid; e < 3 * box_nodes; e += BS) box[e] = 0.0;
-    for (int b = tid; b <= kMaxPlanes; b += BS) pcount[b] = 0;
+    // the spread's scratch starts at zero: the row masks and the node sums
+    for (int e = tid; e < scratch_bytes / 8; e += BS) region[e] = 0.0;
   }
   __syncthreads();
   use_pk = REL && !bad && !farpk;
   const int o0 = bmin[0], o1 = bmin[1], o2 = bmin[2];
   const int s0 = bmax[0] - bmin[0] + 2, s1 = bmax[1] - bmin[1] + 2, s2 = bmax[2] - bmin[2] + 2;
-  const int64_t plane = (int64_t)s1 * s2;
-  // the box is spread in slabs of whole x-planes when it does not fit at once;
-  // only a cell whose single x-plane does not fit uses global atomics per vertex
-  const bool direct = bad || s0 <= 0 || plane > box_nodes;
+  // Only the nodes in some vertex's support get a sum: a mask of 64 z-nodes per
+  // (x, y) row of the box says which, and a node's place is the number of marked
+  // nodes before it.  An RBC's surface touches ~1290 of the up to 5832 nodes of
+  // its box and fits in two passes of ~680 sums (a WBC's 2210 in four), where
+  // slabs of the whole box took one pass per x-plane (18 passes of ~70 vertices
+  // on 256 threads, two barriers each).  With the supports' short forms above:
+  // the 15.5k-RBC suspension's step 3.23 -> 2.99 ms in FP32 and 2.88 -> 2.85 ms
+  // (half the box) in FP64, a lone RBC 73 -> 58 us with everything in one pass.
+  const int zw = (s2 + 63) >> 6;
+  const bool sane = !bad && s0 > 0 && s0 <= 4096 && s1 <= 4096 && s2 <= 65536;
+  const int64_t nrows = sane ? (int64_t)s0 * s1 * zw : 0;
+  // per row a 64-bit mask and a first place, per sum 3 doubles and its node
+  const bool direct = !sane || 12 * nrows + 28 * 64 > scratch_bytes;
   const int64_t S = L.stride;
   auto spread_force = [&](int64_t i, double& f0, double& f1, double& f2) {
     if (incomplete && (V.flag[i] & VFLAG_REMOVED)) {
@@ -432,99 +470,116 @@ __device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev
       spread_force(i, f0, f1, f2);
       const SW g0 = (SW)f0, g1 = (SW)f1, g2 = (SW)f2;
       SupportT<SW> sp;
-      ibm_support(pos_x(k), pos_y(k), pos_z(k), L, type, sp);
+      support_of(k, sp);
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         if (sp.w[q] == SW(0)) continue;
         const int64_t n = sp.idx[q];
-        atomic_add(&Fnext[n], (R)spread_term((double)(g0 * sp.w[q]), L));
-        atomic_add(&Fnext[S + n], (R)spread_term((double)(g1 * sp.w[q]), L));
-        atomic_add(&Fnext[2 * S + n], (R)spread_term((double)(g2 * sp.w[q]), L));
+        atomic_add(&Fnext[n], (R)spread_term<R>((double)(g0 * sp.w[q]), L));
+        atomic_add(&Fnext[S + n], (R)spread_term<R>((double)(g1 * sp.w[q]), L));
+        atomic_add(&Fnext[2 * S + n], (R)spread_term<R>((double)(g2 * sp.w[q]), L));
       }
     }
     return;
   }
-  const int sx = (int)std::min<int64_t>(s0, box_nodes / plane);  // x-planes per slab
-  // With several slabs, the vertices are bucketed by the x-plane of their
-  // support's low corner (a vertex adds to that plane and the next), so a slab
-  // visits only the vertices that reach it.
-  const bool bucketed = sx < s0 && s0 <= kMaxPlanes && nv <= 65535;
-  if (bucketed) {
-    for (int k = tid; k < nv; k += BS) atomicAdd(&pcount[(int)floor(pos_x(k)) - o0], 1);
-    __syncthreads();
-    if (tid < 64) {
-      // exclusive prefix sum of the s0 + 1 <= 65 plane counts over wavefront 0;
-      // the counts become the insertion cursors
-      const int c = tid <= s0 ? pcount[tid] : 0;
-      int inc = c;
+  const int rows = (int)nrows;
+  const int cap = (scratch_bytes - 12 * rows) / 28;
+  unsigned long long* const mask = reinterpret_cast<unsigned long long*>(region);
+  double* const box = region + rows;
+  uint32_t* const place = reinterpret_cast<uint32_t*>(box + 3 * cap);
+  uint32_t* const node = place + rows;
+  // lanes of one wavefront take vertices ~nv/64 apart (fewer LDS same-address operations)
+  const int per = (nv + 63) / 64;
+  for (int k = tid; k < 64 * per; k += BS) {
+    const int vtx = (k & 63) * per + (k >> 6);
+    if (vtx >= nv) continue;
+    int n0[3];
+    low_node(vtx, n0);
+    const int lz = n0[2] - o2;
+    const int r = (n0[1] - o1 + s1 * (n0[0] - o0)) * zw + (lz >> 6), bit = lz & 63;
 #pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(inc, o);
-        if (tid >= o) inc += y;
-      }
-      if (tid <= s0) {
-        pstart[tid] = inc - c;
-        pcount[tid] = inc - c;
-      }
-      if (tid == 63 && s0 == 64) {
-        pstart[64] = inc;
-        pcount[64] = inc;
-      }
+    for (int q = 0; q < 4; ++q) {
+      const int rq = r + ((q >> 1) * s1 + (q & 1)) * zw;
+      atomicOr(&mask[rq], 3ull << bit);
+      if (bit == 63) atomicOr(&mask[rq + 1], 1ull);
     }
+  }
+  __syncthreads();
+  // each row's first place: an exclusive prefix sum of the rows' node counts
+  int total = 0;
+  for (int r0 = 0; r0 < rows; r0 += BS) {
+    const int r = r0 + tid;
+    const int c = r < rows ? __popcll(mask[r]) : 0;
+    int inc = c;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(inc, o);
+      if ((tid & 63) >= o) inc += y;
+    }
+    if ((tid & 63) == 63) wsum[tid >> 6] = inc;
     __syncthreads();
-    for (int k = tid; k < nv; k += BS) vlist[atomicAdd(&pcount[(int)floor(pos_x(k)) - o0], 1)] = (uint16_t)k;
-    __syncthreads();
+    int before = total;
+#pragma unroll
+    for (int w = 0; w < BS / 64; ++w) {
+      if (w < (tid >> 6)) before += wsum[w];
+      total += wsum[w];
+    }
+    if (r < rows) place[r] = (uint32_t)(before + inc - c);
+    if (r0 + BS < rows) __syncthreads();
   }
   const int dims[3] = {L.nx, L.ny, L.nz};
-  for (int xs = 0; xs < s0; xs += sx) {
-    const int nxp = std::min(sx, s0 - xs);
-    // the slab fits the box (plane <= box_nodes), so 32-bit indices suffice
-    const int total = nxp * (int)plane;
-    // the vertices to visit: a range of the bucketed list, or all of them
-    const int first = bucketed ? pstart[max(xs - 1, 0)] : 0;
-    const int count = bucketed ? pstart[min(xs + nxp, s0)] - first : nv;
-    const int per = (count + 63) / 64;
+  auto wrapped = [&](int a, int c) -> uint32_t { return (c >= 0 && c < dims[a]) ? (uint32_t)c : (uint32_t)wrap_node((double)c, dims[a]); };
+  for (int p0 = 0; p0 < total; p0 += cap) {
+    const int count = min(cap, total - p0);
+    // the nodes of this pass's places (a thread's rows are those whose place it wrote)
+    for (int r = tid; r < rows; r += BS) {
+      unsigned long long m = mask[r];
+      int j = (int)place[r] - p0;
+      if (j >= count || j + __popcll(m) <= 0) continue;
+      const unsigned xy = zw == 1 ? (unsigned)r : (unsigned)r / (unsigned)zw;
+      const unsigned lx = xy / (unsigned)s1, ly = xy - lx * (unsigned)s1;
+      const int z = o2 + 64 * (r - (int)xy * zw);
+      const uint32_t at = (uint32_t)L.nz * (wrapped(1, o1 + (int)ly) + (uint32_t)L.ny * wrapped(0, o0 + (int)lx));
+      for (; m; m &= m - 1, ++j)
+        if (j >= 0 && j < count) node[j] = at + wrapped(2, z + __builtin_ctzll(m));
+    }
+    __syncthreads();
     for (int k = tid; k < 64 * per; k += BS) {
-      // lanes of one wavefront take vertices ~count/64 apart (fewer LDS same-address adds)
-      const int j = (k & 63) * per + (k >> 6);
-      if (j >= count) continue;
-      const int vtx = bucketed ? (int)vlist[first + j] : j;
+      const int vtx = (k & 63) * per + (k >> 6);
+      if (vtx >= nv) continue;
+      SupportT<SW> sp;
+      support_of(vtx, sp);
+      const int lz = sp.lo[2] - o2, bit = lz & 63;
+      const int r = (sp.lo[1] - o1 + s1 * (sp.lo[0] - o0)) * zw + (lz >> 6);
       double f0, f1, f2;
       spread_force(base + vtx, f0, f1, f2);
       const SW g0 = (SW)f0, g1 = (SW)f1, g2 = (SW)f2;
-      SupportT<SW> sp;
-      ibm_support(pos_x(vtx), pos_y(vtx), pos_z(vtx), L, type, sp);
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int lx = sp.lo[0] + (q >> 2) - o0 - xs;
-        if (sp.w[q] == SW(0) || lx < 0 || lx >= nxp) continue;
-        const int e = (sp.lo[2] + (q & 1) - o2) + s2 * ((sp.lo[1] + ((q >> 1) & 1) - o1) + s1 * lx);
-        lds_add(&box[e], spread_term((double)(g0 * sp.w[q]), L));
-        lds_add(&box[total + e], spread_term((double)(g1 * sp.w[q]), L));
-        lds_add(&box[2 * total + e], spread_term((double)(g2 * sp.w[q]), L));
+      for (int q = 0; q < 8; q += 2) {
+        const int rq = r + ((q >> 2) * s1 + ((q >> 1) & 1)) * zw;
+        // the node at z and the next place, z + 1
+        const int e = (int)place[rq] - p0 + __popcll(mask[rq] & ((1ull << bit) - 1ull));
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          if ((unsigned)(e + h) >= (unsigned)count || sp.w[q + h] == SW(0)) continue;
+          lds_add(&box[e + h], spread_term<R>((double)(g0 * sp.w[q + h]), L));
+          lds_add(&box[cap + e + h], spread_term<R>((double)(g1 * sp.w[q + h]), L));
+          lds_add(&box[2 * cap + e + h], spread_term<R>((double)(g2 * sp.w[q + h]), L));
+        }
       }
     }
     __syncthreads();
-    const unsigned us1 = (unsigned)s1, us2 = (unsigned)s2;
-    for (int e = tid; e < total; e += BS) {
-      const double a = box[e], b = box[total + e], cz = box[2 * total + e];
-      if (a == 0.0 && b == 0.0 && cz == 0.0) continue;
-      box[e] = 0.0;  // zero for the next slab, whose box is no larger
-      box[total + e] = 0.0;
-      box[2 * total + e] = 0.0;
-      const unsigned r = (unsigned)e / us2;
-      const int lz = (int)((unsigned)e - r * us2);
-      const unsigned r2 = r / us1;
-      const int ly = (int)(r - r2 * us1), lx = (int)r2;
-      const int64_t g[3] = {(int64_t)o0 + xs + lx, (int64_t)o1 + ly, (int64_t)o2 + lz};
-      int64_t wc[3];
-      for (int q = 0; q < 3; ++q) wc[q] = (g[q] >= 0 && g[q] < dims[q]) ? g[q] : wrap_mod(g[q], dims[q]);
-      const int64_t n = wc[2] + (int64_t)L.nz * (wc[1] + (int64_t)L.ny * wc[0]);
+    for (int j = tid; j < count; j += BS) {
+      const double a = box[j], b = box[cap + j], c = box[2 * cap + j];
+      box[j] = 0.0;  // zero for the next pass
+      box[cap + j] = 0.0;
+      box[2 * cap + j] = 0.0;
+      const int64_t n = node[j];
       if (a != 0.0) atomic_add(&Fnext[n], (R)a);
       if (b != 0.0) atomic_add(&Fnext[S + n], (R)b);
-      if (cz != 0.0) atomic_add(&Fnext[2 * S + n], (R)cz);
+      if (c != 0.0) atomic_add(&Fnext[2 * S + n], (R)c);
     }
-    __syncthreads();  // the box is zero again for the next slab
+    if (p0 + cap < total) __syncthreads();  // the sums are zero and the nodes free again
   }
 }
 
@@ -656,6 +711,7 @@ hipError_t launch_cell_step(hipStream_t s, const VertexDev& V, const TypeDev& T,
       HC_CELL(HC_MODEL_RBC, 256)
       break;
     case HC_MODEL_PLT:
+      if (block >= 256) HC_CELL(HC_MODEL_PLT, 256)
       HC_CELL(HC_MODEL_PLT, 64)
       break;
     case HC_MODEL_WBC:
@@ -725,8 +781,6 @@ hipError_t launch_cell_step_multi(hipStream_t s, const TypeDev& T, const CellCas
       HC_CELL(HC_MODEL_RBC, 256)
       return e;
     case HC_MODEL_PLT:
-      // fewer platelets than compute units (the caller passes block 1024 then):
-      // four waves per platelet shorten its box clear and flush
       if (block >= 256) HC_CELL(HC_MODEL_PLT, 256)
       HC_CELL(HC_MODEL_PLT, 64)
       return e;

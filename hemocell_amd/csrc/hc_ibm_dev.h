@@ -34,66 +34,97 @@ struct SupportT {
 };
 using Support = SupportT<double>;
 
-__device__ __forceinline__ int64_t wrap_far(int64_t c, int n) {
-  const double q = floor((double)c / (double)n);
-  return c - (int64_t)q * n;
+// Coordinate of node fl (an integer, |fl| < 2^53) on a periodic axis of size n.
+__device__ __forceinline__ int wrap_node(double fl, int n) {
+  double m = fl - (double)n * floor(fl / (double)n);
+  if (m < 0.0) m += (double)n;
+  if (m >= (double)n) m -= (double)n;
+  return (int)m;
+}
+
+// Node indices and normalised weights from the low corner n0 and the hat values
+// q of each axis.  A support inside the domain (all but the vertices at a domain
+// face) is one index and three strides; otherwise the axes that leave it are
+// wrapped or, closed, lose the hat value beyond the face: `fl(a)` gives the low
+// corner as a double there (positions far outside do not fit an int).
+template <typename W, typename FL>
+__device__ __forceinline__ void finish_support(const int (&n0)[3], W (&q)[3][2], bool finite, FL fl,
+                                               const LatticeDev& L, const uint8_t* __restrict__ type, SupportT<W>& s) {
+  const int dims[3] = {L.nx, L.ny, L.nz};
+  int w0[3], step[3];
+  bool inside = finite;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    s.lo[a] = w0[a] = n0[a];
+    step[a] = 1;
+    inside = inside && (unsigned)n0[a] < (unsigned)(dims[a] - 1);
+  }
+  if (!inside) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      int w[2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const double node = finite ? fl(a) + (double)k : -1.0;
+        if (node >= 0.0 && node < (double)dims[a]) {
+          w[k] = (int)node;
+        } else if (finite && L.periodic[a]) {
+          w[k] = wrap_node(node, dims[a]);
+        } else {
+          w[k] = 0;
+          q[a][k] = W(0);
+        }
+      }
+      w0[a] = w[0];
+      step[a] = w[1] - w[0];
+    }
+  }
+  const uint32_t dz = (uint32_t)step[2], dy = (uint32_t)step[1] * (uint32_t)L.nz,
+                 dx = (uint32_t)step[0] * (uint32_t)(L.ny * L.nz);
+  const uint32_t n = (uint32_t)w0[2] + (uint32_t)L.nz * ((uint32_t)w0[1] + (uint32_t)L.ny * (uint32_t)w0[0]);
+  W total = W(0);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    s.idx[k] = n + ((k & 4) ? dx : 0u) + ((k & 2) ? dy : 0u) + ((k & 1) ? dz : 0u);
+    s.w[k] = q[0][k >> 2] * q[1][(k >> 1) & 1] * q[2][k & 1];
+  }
+  if (type) {
+    uint8_t t[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) t[k] = type[s.idx[k]];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (t[k] != HC_NODE_FLUID) s.w[k] = W(0);
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) total += s.w[k];
+  const W coeff = W(1) / total;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) s.w[k] = s.w[k] != W(0) ? s.w[k] * coeff : W(0);
 }
 
 template <typename W>
 __device__ __forceinline__ void ibm_support(double p0, double p1, double p2, const LatticeDev& L,
                                             const uint8_t* __restrict__ type, SupportT<W>& s) {
   const double p[3] = {p0, p1, p2};
-  const int dims[3] = {L.nx, L.ny, L.nz};
   W q[3][2];
-  int wi[3][2];
-  bool ok[3][2];
+  int n0[3];
   bool finite = true;
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
-    finite &= fabs(p[a]) < 1.0e15;
-    const double fl = finite ? floor(p[a]) : 0.0;
-    const int64_t n0 = (int64_t)fl;
-    s.lo[a] = (int)n0;
+    finite = finite && fabs(p[a]) < 1.0e15;
+    const double fl = floor(p[a]);
+    n0[a] = (int)fl;
     if (std::is_same<W, float>::value) {
       const W d = (W)(p[a] - fl);  // in [0, 1)
       q[a][0] = W(1) - d;
       q[a][1] = d;
-    }
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const int64_t node = n0 + k;
-      if (!std::is_same<W, float>::value) q[a][k] = (W)fmax(1.0 - fabs(p[a] - (double)node), 0.0);
-      if (node >= 0 && node < dims[a]) {
-        wi[a][k] = (int)node;
-        ok[a][k] = true;
-      } else if (L.periodic[a]) {
-        wi[a][k] = (int)(node == -1 ? dims[a] - 1 : (node == dims[a] ? 0 : wrap_far(node, dims[a])));
-        ok[a][k] = true;
-      } else {
-        wi[a][k] = 0;
-        ok[a][k] = false;
-      }
+    } else {
+      q[a][0] = (W)fmax(1.0 - fabs(p[a] - fl), 0.0);
+      q[a][1] = (W)fmax(1.0 - fabs(p[a] - (fl + 1.0)), 0.0);
     }
   }
-  W total = W(0);
-#pragma unroll
-  for (int ix = 0; ix < 2; ++ix)
-#pragma unroll
-    for (int iy = 0; iy < 2; ++iy)
-#pragma unroll
-      for (int iz = 0; iz < 2; ++iz) {
-        const int slot = ix * 4 + iy * 2 + iz;
-        const uint32_t n = (uint32_t)wi[2][iz] + (uint32_t)L.nz * ((uint32_t)wi[1][iy] + (uint32_t)L.ny * (uint32_t)wi[0][ix]);
-        const W ww = q[0][ix] * q[1][iy] * q[2][iz];
-        bool keep = finite && ok[0][ix] && ok[1][iy] && ok[2][iz] && ww != W(0);
-        if (keep && type) keep = type[n] == HC_NODE_FLUID;
-        s.idx[slot] = n;
-        s.w[slot] = keep ? ww : W(0);
-        total += s.w[slot];
-      }
-  const W coeff = W(1) / total;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) s.w[k] = s.w[k] != W(0) ? s.w[k] * coeff : W(0);
+  finish_support(n0, q, finite, [&](int a) { return floor(p[a]); }, L, type, s);
 }
 
 // One force contribution to the spread: rounded to a multiple of L.spread_q when
@@ -101,7 +132,9 @@ __device__ __forceinline__ void ibm_support(double p0, double p1, double p2, con
 // exact and rint is the only rounding; the sums of such multiples stay exact
 // (hence independent of the order of the adds) while they are below 2^53
 // spread_q in magnitude.
+template <typename R>
 __device__ __forceinline__ double spread_term(double v, const LatticeDev& L) {
+  if (std::is_same<R, float>::value) return v;  // FP64 only
   return L.spread_q > 0.0 ? rint(v * L.spread_inv_q) * L.spread_q : v;
 }
 
