@@ -84,6 +84,8 @@ struct hc_ctx {
   uint8_t* vflag = nullptr;  // per vertex: VFLAG_REMOVED
   int64_t* d_cell_base = nullptr;
   int32_t* d_cell_nv = nullptr;
+  int* d_box = nullptr;        // support box per cell (VertexDev::box)
+  double box_nodes = 0;        // nodes in the cells' support boxes, from the rest meshes
   bool cells_dirty = true;
   int lds_limit = 65536;        // dynamic LDS per workgroup available on the device
   int lds_device = 65536;       // LDS per workgroup of the device (static + dynamic)
@@ -207,7 +209,7 @@ hc_status dalloc(hc_ctx* ctx, void** p, size_t bytes, const char* what) {
   return HC_OK;
 }
 
-VertexDev vdev(hc_ctx* c) { return VertexDev{c->x, c->v, c->fv, c->frep, c->fbr, c->nv, c->vcap, c->vflag}; }
+VertexDev vdev(hc_ctx* c) { return VertexDev{c->x, c->v, c->fv, c->frep, c->fbr, c->nv, c->vcap, c->vflag, c->d_box}; }
 
 void prof_begin(hc_ctx* c, int stage, hipEvent_t* start) {
   *start = nullptr;
@@ -381,6 +383,17 @@ hc_status sync_cells(hc_ctx* ctx) {
     std::vector<int32_t> cnv(nc);
     for (size_t c = 0; c < nc; ++c) cnv[c] = ctx->types[ctx->cell_type[c]]->host.nv;
     if (nc) HC_TRY(hipMemcpy(ctx->d_cell_nv, cnv.data(), sizeof(int32_t) * nc, hipMemcpyHostToDevice), "hipMemcpy");
+  }
+  if (ctx->d_box) hipFree(ctx->d_box);
+  ctx->d_box = nullptr;
+  if ((s = dalloc(ctx, (void**)&ctx->d_box, sizeof(int) * kBoxInts * std::max<size_t>(nc, 1), "cell boxes")) != HC_OK)
+    return s;
+  ctx->box_nodes = 0;
+  for (size_t c = 0; c < nc; ++c) {
+    // a cell turns: its largest extent on every axis
+    const TypeHost& h = ctx->types[ctx->cell_type[c]]->host;
+    const double side = h.extent + 3.0;
+    ctx->box_nodes += side * side * side;
   }
   // Launch order: the cells of a type by the 8-node tile of their centre, tiles in
   // the lattice's x, y, z order (z fastest, as the node index runs).  Workgroups
@@ -697,6 +710,25 @@ bool mixed_cell_step(hc_ctx* ctx, int do_interp, hc_status& st) {
   return true;
 }
 
+// Whether the fused step needs the velocity field on the cells' boxes only: they
+// cover less than half of the lattice (a box's short rows read whole cache lines,
+// so that at half of the nodes both passes move about the same), and the spread
+// of the current positions noted them (HC_SPREAD=vertex does not).
+bool velocity_on_boxes(const hc_ctx* ctx) {
+  return ctx->spread_per_cell && ctx->box_nodes < 0.5 * (double)ctx->L.N;
+}
+
+BoxCase box_case(hc_ctx* c, int cur) {
+  BoxCase b{};
+  b.f = c->f;
+  b.Fcur = c->Fibm[cur];
+  b.uf = c->ufield;
+  b.box = c->d_box;
+  b.L = c->L;
+  for (int k = 0; k < 3; ++k) b.g[k] = c->g[k];
+  return b;
+}
+
 template <typename R>
 hc_status do_cell_step(hc_ctx* ctx, int do_interp) {
   hipEvent_t ev;
@@ -885,9 +917,14 @@ hc_status one_step(hc_ctx* ctx) {
     if (do_interp) {
       hipEvent_t e2;
       prof_begin(ctx, HC_PROF_INTERP, &e2);
-      HC_TRY(launch_velocity_field<R>(ctx->stream, (const R*)ctx->f, (const R*)ctx->Fibm[ctx->cur], (R*)ctx->ufield,
-                                      ctx->L, ctx->phase, ctx->general, ctx->g),
-             "velocity_field");
+      if (velocity_on_boxes(ctx))
+        HC_TRY(launch_velocity_boxes<R>(ctx->stream, box_case(ctx, ctx->cur), (int)ctx->cell_base.size(), ctx->phase,
+                                        ctx->general),
+               "velocity_field");
+      else
+        HC_TRY(launch_velocity_field<R>(ctx->stream, (const R*)ctx->f, (const R*)ctx->Fibm[ctx->cur], (R*)ctx->ufield,
+                                        ctx->L, ctx->phase, ctx->general, ctx->g),
+               "velocity_field");
       prof_end(ctx, HC_PROF_INTERP, e2);
     }
     if ((s = do_cell_step<R>(ctx, do_interp)) != HC_OK) return s;
@@ -939,6 +976,8 @@ std::vector<unsigned char> launch_signature(const hc_ctx* c) {
   put(v, c->nv);
   put(v, c->vcap);
   put(v, c->d_cell_base);
+  put(v, c->d_box);
+  put(v, c->box_nodes);
   put(v, c->d_extra_dense);
   put(v, c->d_wall_hits);
   put(v, c->lds_limit);
@@ -1086,7 +1125,7 @@ hc_status batch_impl(hc_ctx* const* cs, int n, int nsteps) {
   }
   // descriptors for the two parities of the step counter
   struct Group {
-    int kind;  // 0 collide, 1 velocity field, 2 cells
+    int kind;  // 0 collide, 1 velocity field, 2 cells, 3 velocity field on cell boxes
     int a, b, c;
     size_t offset;
     int count;
@@ -1099,6 +1138,7 @@ hc_status batch_impl(hc_ctx* const* cs, int n, int nsteps) {
     // collide: key (odd, general, vel)
     std::map<std::tuple<int, int, int>, std::vector<LatCase>> lat;
     std::map<std::tuple<int, int>, std::vector<VelCase>> vel;
+    std::map<std::tuple<int, int>, std::vector<BoxCase>> boxes;
     std::map<std::tuple<int, int, int>, std::vector<CellCase>> cel;
     std::map<std::tuple<int, int, int>, TypeDev> cel_t;
     for (int i = 0; i < n; ++i) {
@@ -1115,19 +1155,29 @@ hc_status batch_impl(hc_ctx* const* cs, int n, int nsteps) {
       std::memcpy(lc.a.wall_u, c->wall_u, sizeof(lc.a.wall_u));
       const int vflag = c->general && c->n_vel > 0 && c->fuse_vel;
       lat[std::make_tuple(phase, (int)c->general, vflag)].push_back(lc);
-      VelCase vc{};
-      vc.f = c->f;
-      vc.Fcur = c->Fibm[cur];
-      vc.uf = c->ufield;
-      vc.L = c->L;
-      for (int k = 0; k < 3; ++k) vc.g[k] = c->g[k];
-      vel[std::make_tuple(phase ^ 1, (int)c->general)].push_back(vc);
+      const auto vkey = std::make_tuple(phase ^ 1, (int)c->general);
+      if (velocity_on_boxes(c)) {
+        BoxCase bc = box_case(c, cur);
+        for (size_t k = 0; k < c->cell_base.size(); ++k) {
+          bc.box = c->d_box + kBoxInts * (int64_t)k;
+          boxes[vkey].push_back(bc);
+        }
+      } else {
+        VelCase vc{};
+        vc.f = c->f;
+        vc.Fcur = c->Fibm[cur];
+        vc.uf = c->ufield;
+        vc.L = c->L;
+        for (int k = 0; k < 3; ++k) vc.g[k] = c->g[k];
+        vel[vkey].push_back(vc);
+      }
       for (size_t k = 0; k < c->cell_base.size(); ++k) {
         const TypeBufs& tb = *c->types[(size_t)c->cell_type[k]];
         CellCase cc{};
         cc.V = vdev(c);
         cc.T = tb.dev;
         cc.base = c->cell_base[k];
+        cc.box = c->d_box + kBoxInts * (int64_t)k;
         cc.uf = c->ufield;
         cc.type = c->type;
         cc.L = c->L;
@@ -1167,6 +1217,12 @@ hc_status batch_impl(hc_ctx* const* cs, int n, int nsteps) {
       align();
       Group g{1, std::get<0>(kv.first), std::get<1>(kv.first), 0, bytes.size(), (int)kv.second.size(), blocks,
               TypeDev{}};
+      append_bytes(bytes, kv.second);
+      groups[p].push_back(g);
+    }
+    for (auto& kv : boxes) {
+      align();
+      Group g{3, std::get<0>(kv.first), std::get<1>(kv.first), 0, bytes.size(), (int)kv.second.size(), 0, TypeDev{}};
       append_bytes(bytes, kv.second);
       groups[p].push_back(g);
     }
@@ -1212,6 +1268,9 @@ hc_status batch_impl(hc_ctx* const* cs, int n, int nsteps) {
       } else if (g.kind == 1) {
         HC_TRY(launch_velocity_field_multi<R>(lead->stream, (const VelCase*)(base + g.offset), g.count, g.blocks,
                                               g.a, g.b != 0),
+               "batched velocity_field");
+      } else if (g.kind == 3) {
+        HC_TRY(launch_velocity_boxes_multi<R>(lead->stream, (const BoxCase*)(base + g.offset), g.count, g.a, g.b != 0),
                "batched velocity_field");
       }
     }
@@ -1485,7 +1544,7 @@ void hc_destroy(hc_ctx* ctx) {
   hipSetDevice(ctx->device);
   hipStreamSynchronize(ctx->stream);
   void* ps[] = {ctx->d_queue, ctx->d_types, ctx->d_head,
-                ctx->f, ctx->Fibm[0], ctx->Fibm[1], ctx->ufield, ctx->d_cell_nv, ctx->d_extra_dense, ctx->type, ctx->vel_nodes, ctx->x, ctx->v, ctx->fv, ctx->frep, ctx->bend,
+                ctx->f, ctx->Fibm[0], ctx->Fibm[1], ctx->ufield, ctx->d_cell_nv, ctx->d_box, ctx->d_extra_dense, ctx->type, ctx->vel_nodes, ctx->x, ctx->v, ctx->fv, ctx->frep, ctx->bend,
                 ctx->fbr, ctx->vflag, ctx->d_bflag, ctx->d_cell_base, ctx->d_extra_ids, ctx->d_extra_f, ctx->d_wall_hits, ctx->d_flag,
                 ctx->d_visc, ctx->d_stamp, ctx->d_xold, ctx->d_le, ctx->d_batch[0], ctx->d_batch[1]};
   for (void* p : ps)
@@ -1643,6 +1702,14 @@ hc_status hc_add_cell_type(hc_ctx* ctx, int model, int nv, int nt, const int32_t
   T.nt = nt;
   T.tri.assign(triangles, triangles + 3 * nt);
   T.rest.assign(rest, rest + 3 * nv);
+  for (int a = 0; a < 3; ++a) {
+    double lo = rest[a], hi = rest[a];
+    for (int k = 1; k < nv; ++k) {
+      lo = std::min(lo, rest[3 * k + a]);
+      hi = std::max(hi, rest[3 * k + a]);
+    }
+    T.extent = std::max(T.extent, hi - lo);
+  }
   if (n_inner > 0) T.inner.assign(inner, inner + 2 * n_inner);
   T.p = *params;
   T.timescale = timescale > 0 ? timescale : 1;

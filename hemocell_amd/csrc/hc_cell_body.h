@@ -48,7 +48,7 @@ using MechT = typename std::conditional<std::is_same<R, float>::value && STAGED 
 // workgroup needs LDS only for the spread box and fits beside the many small
 // workgroups of another cell type running at the same time.
 template <typename R, int MODEL, int BS, bool STAGED, bool GPOS>
-__device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev& T, const int64_t base,
+__device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev& T, const int64_t base, int* cell_box,
                                                const R* __restrict__ uf, const uint8_t* __restrict__ type,
                                                const LatticeDev& L, R* __restrict__ Fnext,
                                                const double* __restrict__ extra, double* __restrict__ scratch,
@@ -433,6 +433,7 @@ __device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev
   }
   __syncthreads();
   use_pk = REL && !bad && !farpk;
+  if (tid == 0) write_box(cell_box, bmin, bmax, bad != 0);
   const int o0 = bmin[0], o1 = bmin[1], o2 = bmin[2];
   const int s0 = bmax[0] - bmin[0] + 2, s1 = bmax[1] - bmin[1] + 2, s2 = bmax[2] - bmin[2] + 2;
   // Only the nodes in some vertex's support get a sum: a mask of 64 z-nodes per
@@ -590,7 +591,8 @@ __global__ __launch_bounds__(BS) void k_cell_step(VertexDev V, TypeDev T, const 
                                                   const double* __restrict__ extra, double* __restrict__ scratch,
                                                   double f_limit, int flags, int box_nodes,
                                                   unsigned long long* wall_hits) {
-  cell_step_body<R, MODEL, BS, STAGED, GPOS>(V, T, cell_base[cells[blockIdx.x]], uf, type, L, Fnext, extra, scratch,
+  cell_step_body<R, MODEL, BS, STAGED, GPOS>(V, T, cell_base[cells[blockIdx.x]],
+                                             V.box ? V.box + kBoxInts * (int64_t)cells[blockIdx.x] : nullptr, uf, type, L, Fnext, extra, scratch,
                                              f_limit, flags, box_nodes, wall_hits);
 }
 
@@ -598,7 +600,7 @@ __global__ __launch_bounds__(BS) void k_cell_step(VertexDev V, TypeDev T, const 
 template <typename R, int MODEL, int BS, bool STAGED, bool GPOS>
 __global__ __launch_bounds__(BS) void k_cell_step_multi(const CellCase* __restrict__ cs, int box_nodes) {
   const CellCase& c = cs[blockIdx.x];
-  cell_step_body<R, MODEL, BS, STAGED, GPOS>(c.V, c.T, c.base, (const R*)c.uf, c.type, c.L, (R*)c.Fnext, c.extra,
+  cell_step_body<R, MODEL, BS, STAGED, GPOS>(c.V, c.T, c.base, c.box, (const R*)c.uf, c.type, c.L, (R*)c.Fnext, c.extra,
                                              c.scratch, c.f_limit, c.flags, box_nodes, c.wall_hits);
 }
 
@@ -622,14 +624,15 @@ __global__ __launch_bounds__(kMixedBlock) void k_cell_step_mixed(
     const int2 e = queue[q];
     const TypeDev& T = types[e.y];
     const int64_t base = cell_base[e.x];
+    int* const box = V.box ? V.box + kBoxInts * (int64_t)e.x : nullptr;
     if (T.model == HC_MODEL_RBC)
-      cell_step_body<R, HC_MODEL_RBC, kMixedBlock, true, false>(V, T, base, uf, type, L, Fnext, extra, scratch,
+      cell_step_body<R, HC_MODEL_RBC, kMixedBlock, true, false>(V, T, base, box, uf, type, L, Fnext, extra, scratch,
                                                                  f_limit, A.flags[e.y], A.box_nodes[e.y], wall_hits);
     else if (T.model == HC_MODEL_PLT)
-      cell_step_body<R, HC_MODEL_PLT, kMixedBlock, true, false>(V, T, base, uf, type, L, Fnext, extra, scratch,
+      cell_step_body<R, HC_MODEL_PLT, kMixedBlock, true, false>(V, T, base, box, uf, type, L, Fnext, extra, scratch,
                                                                  f_limit, A.flags[e.y], A.box_nodes[e.y], wall_hits);
     else
-      cell_step_body<R, HC_MODEL_WBC, kMixedBlock, false, true>(V, T, base, uf, type, L, Fnext, extra, scratch,
+      cell_step_body<R, HC_MODEL_WBC, kMixedBlock, false, true>(V, T, base, box, uf, type, L, Fnext, extra, scratch,
                                                                  f_limit, A.flags[e.y], A.box_nodes[e.y], wall_hits);
     __syncthreads();  // the next cell reuses the LDS
   }

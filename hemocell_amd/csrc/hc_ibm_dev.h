@@ -176,6 +176,15 @@ __device__ __forceinline__ void block_bounds(const int (&lmin)[3], const int (&l
   }
 }
 
+// one thread's note of a cell's support box (VertexDev::box)
+__device__ __forceinline__ void write_box(int* box, const int* bmin, const int* bmax, bool bad) {
+  if (!box) return;
+  for (int a = 0; a < 3; ++a) {
+    box[a] = bmin[a];
+    box[3 + a] = bad || bmax[a] < bmin[a] ? -1 : bmax[a] - bmin[a] + 2;
+  }
+}
+
 __device__ __forceinline__ void atomic_add(float* p, float v) { unsafeAtomicAdd(p, v); }
 __device__ __forceinline__ void atomic_add(double* p, double v) { unsafeAtomicAdd(p, v); }
 

@@ -31,6 +31,7 @@ struct TypeHost {
   std::vector<int32_t> nring;       // nv
   std::vector<int32_t> inner;       // ni*2
   std::vector<double> edge_len_eq, edge_angle_eq, tri_area_eq, patch_dist_eq, inner_len_eq;
+  double extent = 0;  // largest axis extent of the rest mesh
   double volume_eq = 0, area_mean_eq = 0, edge_mean_eq = 0, angle_mean_eq = 0;
   // gather lists (CSR): entries per vertex in accumulation order
   std::vector<int32_t> vtri_off, vtri;      // t*4 + corner slot

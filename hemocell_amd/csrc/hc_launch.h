@@ -55,8 +55,13 @@ struct VertexDev {
   // (HemoCellParticleField::advanceParticles); a cell with a removed vertex is
   // incomplete: no mechanics, zero force, its other vertices still drift
   uint8_t* flag;
+  // per cell: the low corner and the size of the box of its vertices' support
+  // nodes, kBoxInts integers, written by the spread of the current positions
+  // (size[0] = -1: positions that have none)
+  int* box;
 };
 constexpr uint8_t VFLAG_REMOVED = 1;
+constexpr int kBoxInts = 8;
 template <typename R>
 hipError_t launch_spread(hipStream_t s, const VertexDev& V, R* Fibm, const uint8_t* type, const LatticeDev& L,
                          double f_limit, int use_repulsion);
@@ -146,12 +151,30 @@ template <typename R>
 hipError_t launch_velocity_field_multi(hipStream_t s, const VelCase* cases, int ncase, uint32_t blocks, int phase,
                                        bool general);
 
+// The velocity field on the support boxes of single cells only (few cells in a
+// large box): one entry per cell.
+struct BoxCase {
+  const void* f;
+  const void* Fcur;
+  void* uf;
+  const int* box;  // the cell's box (VertexDev::box)
+  LatticeDev L;
+  double g[3];
+};
+// one lattice, ncells cells whose boxes follow one another from c.box
+template <typename R>
+hipError_t launch_velocity_boxes(hipStream_t s, const BoxCase& c, int ncells, int phase, bool general);
+// ncells cells of several lattices of one phase and boundary kind
+template <typename R>
+hipError_t launch_velocity_boxes_multi(hipStream_t s, const BoxCase* cases, int ncells, int phase, bool general);
+
 // one cell of a batched cell-step launch (hc_cell.hip): everything the per-type
 // launch passes, for the cell at vertex base `base` of its case
 struct CellCase {
   VertexDev V;
   TypeDev T;
   int64_t base;
+  int* box;  // this cell's entry of V.box
   const void* uf;
   const uint8_t* type;
   LatticeDev L;
