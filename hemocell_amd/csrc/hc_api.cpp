@@ -1125,11 +1125,11 @@ hc_status batch_impl(hc_ctx* const* cs, int n, int nsteps) {
   }
   // descriptors for the two parities of the step counter
   struct Group {
-    int kind;  // 0 collide, 1 velocity field, 2 cells, 3 velocity field on cell boxes
+    int kind;  // 0 collide, 1 velocity field, 2 cells, 3 velocity field on cell boxes, 4 cells of several meshes
     int a, b, c;
     size_t offset;
     int count;
-    uint32_t blocks;
+    uint32_t blocks;  // or the dynamic LDS bytes (kind 4)
     TypeDev T;
   };
   std::vector<Group> groups[2];
@@ -1226,6 +1226,23 @@ hc_status batch_impl(hc_ctx* const* cs, int n, int nsteps) {
       append_bytes(bytes, kv.second);
       groups[p].push_back(g);
     }
+    // no more cells than compute units, of several meshes: one launch for all
+    size_t ncells = 0, dyn = 0;
+    for (const auto& kv : cel) ncells += kv.second.size();
+    bool all = cel.size() > 1 && ncells <= (size_t)lead->n_cu && !lead->cell_block_env;
+    for (auto& kv : cel) {
+      int nodes = 0;
+      all = all && cell_step_all_plan<R>(cel_t[kv.first], spread_box_bytes(lead, std::get<0>(kv.first), true),
+                                         lead->lds_device, &nodes, &dyn);
+      for (CellCase& cc : kv.second) cc.box_nodes = nodes;
+    }
+    if (all) {
+      align();
+      Group g{4, 0, 0, 0, bytes.size(), (int)ncells, (uint32_t)dyn, TypeDev{}};
+      for (auto& kv : cel) append_bytes(bytes, kv.second);
+      groups[p].push_back(g);
+      cel.clear();
+    }
     for (auto& kv : cel) {
       align();
       Group g{2, 0, 0, 0, bytes.size(), (int)kv.second.size(), (uint32_t)kv.second.size(), cel_t[kv.first]};
@@ -1274,6 +1291,10 @@ hc_status batch_impl(hc_ctx* const* cs, int n, int nsteps) {
                "batched velocity_field");
       }
     }
+    for (const Group& g : groups[k & 1])
+      if (g.kind == 4)
+        HC_TRY(launch_cell_step_all<R>(lead->stream, (const CellCase*)(base + g.offset), g.count, g.blocks),
+               "batched cell_step");
     // the cell groups (one per mesh) run side by side: the first on the lead
     // stream, the others on its two side streams, joined before the next step
     int ncell = 0;

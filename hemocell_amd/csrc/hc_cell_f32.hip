@@ -3,6 +3,8 @@
 #include "hc_cell_body.h"
 
 namespace hcg {
+template bool cell_step_all_plan<float>(const TypeDev&, int, int, int*, size_t*);
+template hipError_t launch_cell_step_all<float>(hipStream_t, const CellCase*, int, size_t);
 template hipError_t launch_cell_step_multi<float>(hipStream_t, const TypeDev&, const CellCase*, int, int, int, int);
 template hipError_t launch_cell_step<float>(hipStream_t, const VertexDev&, const TypeDev&, const int32_t*, int,
                                             const int64_t*, const float*, const uint8_t*, const LatticeDev&, float*,

@@ -3,6 +3,8 @@
 #include "hc_cell_body.h"
 
 namespace hcg {
+template bool cell_step_all_plan<double>(const TypeDev&, int, int, int*, size_t*);
+template hipError_t launch_cell_step_all<double>(hipStream_t, const CellCase*, int, size_t);
 template hipError_t launch_cell_step_multi<double>(hipStream_t, const TypeDev&, const CellCase*, int, int, int, int);
 template hipError_t launch_cell_step<double>(hipStream_t, const VertexDev&, const TypeDev&, const int32_t*, int,
                                              const int64_t*, const double*, const uint8_t*, const LatticeDev&, double*,

@@ -183,8 +183,18 @@ struct CellCase {
   double* scratch;
   double f_limit;
   int flags;
+  int box_nodes;  // spread nodes in LDS (launch_cell_step_all)
   unsigned long long* wall_hits;
 };
+// cells of several meshes in one launch (box_nodes set), with the dynamic LDS that
+// cell_step_all_plan asked for over all of them; threads each: the widest block
+// whose registers hold the FP32 bodies, half of it for the FP64 ones
+template <typename R>
+constexpr int all_block() { return sizeof(R) == 4 ? 1024 : 512; }
+template <typename R>
+bool cell_step_all_plan(const TypeDev& T, int box_bytes, int lds_device, int* box_nodes, size_t* dyn);
+template <typename R>
+hipError_t launch_cell_step_all(hipStream_t s, const CellCase* cases, int ncells, size_t dyn);
 // cells of one mesh (T gives the model, vertex count and viscosity for the LDS
 // layout, identical over the cases) from several cases in one launch
 template <typename R>
