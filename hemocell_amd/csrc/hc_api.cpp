@@ -1435,11 +1435,12 @@ hc_status ready_for_step(hc_ctx* ctx) {
 
 template <typename R>
 static hc_status fluid_stats(hc_ctx* ctx, int what, double* out) {
+  const DeviceScope on(ctx->device);
   const int nb = (int)std::min<int64_t>(4096, (ctx->L.N + 255) / 256);
-  double* part = nullptr;
-  R* Fs = nullptr;
-  hc_status s = dalloc(ctx, (void**)&part, sizeof(double) * 4 * nb, "statistics partials");
+  hc_status s = ensure_stage(ctx, sizeof(double) * 4 * nb);
   if (s != HC_OK) return s;
+  double* const h = (double*)ctx->h_stage[0];  // the blocks' partials, written by the kernel
+  R* Fs = nullptr;
   CollideArgs a{};
   a.omega = 1.0 / ctx->tau;
   for (int c = 0; c < 3; ++c) a.g[c] = ctx->g[c];
@@ -1448,11 +1449,9 @@ static hc_status fluid_stats(hc_ctx* ctx, int what, double* out) {
   hipError_t e = hipSuccess;
   if (what == 1) {
     // calculateForceStatistics spreads the vertex forces into a reset field first
-    // (helper/fluidInfo.cpp:117-120): here into a field of its own
-    if ((s = dalloc(ctx, (void**)&Fs, sizeof(R) * 3 * ctx->L.stride, "statistics force field")) != HC_OK) {
-      hipFree(part);
-      return s;
-    }
+    // (helper/fluidInfo.cpp:117-120): here into the velocity field's memory, which
+    // every step fills before it reads it
+    Fs = (R*)ctx->ufield;
     e = launch_fill_zero<R>(ctx->stream, Fs, 3 * ctx->L.stride);
     if (e == hipSuccess && ctx->nv > 0 && sync_cells(ctx) == HC_OK)
       e = launch_spread_cells<R>(ctx->stream, vdev(ctx), Fs, ctx->type, ctx->L, ctx->d_cell_base, ctx->d_cell_nv,
@@ -1460,12 +1459,8 @@ static hc_status fluid_stats(hc_ctx* ctx, int what, double* out) {
                                  std::min(65536, ctx->lds_limit));
   }
   if (e == hipSuccess)
-    e = launch_fluid_stats<R>(ctx->stream, (const R*)ctx->f, Fc, ctx->type, ctx->L, ctx->phase, a, Fs, what, part, nb);
-  std::vector<double> h(4 * (size_t)nb);
-  if (e == hipSuccess) e = hipMemcpyAsync(h.data(), part, sizeof(double) * 4 * nb, hipMemcpyDeviceToHost, ctx->stream);
+    e = launch_fluid_stats<R>(ctx->stream, (const R*)ctx->f, Fc, ctx->type, ctx->L, ctx->phase, a, Fs, what, h, nb);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-  hipFree(part);
-  if (Fs) hipFree(Fs);
   if (e != hipSuccess) return hipfail(ctx, e, "fluid statistics");
   double mn = INFINITY, mx = -INFINITY, sum = 0.0, cnt = 0.0;
   for (int b = 0; b < nb; ++b) {
@@ -2448,17 +2443,24 @@ hc_status hc_get_cell_stats(hc_ctx* ctx, double* volume, double* area, double* c
   const int nc = (int)ctx->cell_base.size();
   if (nc == 0) return HC_OK;
   constexpr int NQ = 15;
+  const DeviceScope on(ctx->device);
+  // the kernels write the pinned slot of a read-back; more cells than it may hold
+  // (8738) go through a device buffer
+  const size_t bytes = sizeof(double) * NQ * nc;
+  const bool direct = bytes <= kStageBytes;
   double* d = nullptr;
-  if ((s = dalloc(ctx, (void**)&d, sizeof(double) * NQ * nc, "cell statistics")) != HC_OK) return s;
+  if ((s = direct ? ensure_stage(ctx, bytes) : dalloc(ctx, (void**)&d, bytes, "cell statistics")) != HC_OK) return s;
+  if (direct) d = (double*)ctx->h_stage[0];
   hipError_t e = hipSuccess;
   for (auto& tp : ctx->types)
     if (e == hipSuccess && tp->ncells)
       e = launch_cell_stats(ctx->stream, vdev(ctx), tp->dev, tp->d_cells, tp->ncells, ctx->d_cell_base, d);
-  std::vector<double> h((size_t)NQ * nc);
-  if (e == hipSuccess) e = hipMemcpyAsync(h.data(), d, sizeof(double) * NQ * nc, hipMemcpyDeviceToHost, ctx->stream);
+  std::vector<double> copy(direct ? 0 : (size_t)NQ * nc);
+  if (e == hipSuccess && !direct) e = hipMemcpyAsync(copy.data(), d, bytes, hipMemcpyDeviceToHost, ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-  hipFree(d);
+  if (!direct) hipFree(d);
   if (e != hipSuccess) return hipfail(ctx, e, "cell statistics");
+  const double* const h = direct ? d : copy.data();
   for (int c = 0; c < nc; ++c) {
     const double* q = &h[(size_t)NQ * c];
     if (volume) volume[c] = q[0];

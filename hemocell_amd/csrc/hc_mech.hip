@@ -141,16 +141,32 @@ __global__ __launch_bounds__(BS) void k_mechanics(VertexDev V, TypeDev T, const 
 // and mean velocity (vertex means), bounding box and the largest vertex-vertex
 // distance.  out[15*c + ...] = vol, area, centroid[3], velocity[3], bbox[6]
 // (xmin, xmax, ymin, ymax, zmin, zmax), stretch.
-template <int BS>
+// STAGED: positions in LDS (nv <= kStatsStaged).  The distances dominate: every
+// pair once, thread i against the next nv/2 vertices round the numbering (equal
+// shares, neighbouring lanes read neighbouring LDS words), compared by their
+// squares, whose largest has the largest root.  From global memory, with a root
+// per pair and the pairs of thread i those above i, 818 RBC took 492 us, now 146.
+constexpr int kStatsStaged = 2700;
+template <int BS, bool STAGED>
 __global__ __launch_bounds__(BS) void k_cell_stats(VertexDev V, TypeDev T, const int32_t* __restrict__ cells,
                                                    const int64_t* __restrict__ cell_base, double* __restrict__ out) {
-  constexpr int NQ = 15;
-  __shared__ double red[NQ][BS];
+  constexpr int NQ = 15, NW = BS / 64;
+  extern __shared__ double sm[];
+  __shared__ double red[NQ][NW];
   const int cell = cells[blockIdx.x];
   const int64_t base = cell_base[cell];
   const int64_t vs = V.vs;
-  const CellView c{V.x + base, V.x + vs + base, V.x + 2 * vs + base};
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, nv = T.nv;
+  CellView c{V.x + base, V.x + vs + base, V.x + 2 * vs + base};
+  if (STAGED) {
+    for (int k = tid; k < nv; k += BS) {
+      sm[k] = c.px[k];
+      sm[nv + k] = c.py[k];
+      sm[2 * nv + k] = c.pz[k];
+    }
+    c = CellView{sm, sm + nv, sm + 2 * nv};
+    __syncthreads();
+  }
   double q[NQ];
   for (int k = 0; k < NQ; ++k) q[k] = 0.0;
   q[8] = q[10] = q[12] = INFINITY;
@@ -168,7 +184,7 @@ __global__ __launch_bounds__(BS) void k_cell_stats(VertexDev V, TypeDev T, const
     q[0] += (1.0 / 6.0) * (-v210 + v120 + v201 - v021 - v102 + v012);
     q[1] += 0.5 * normp(crossp(v1 - v0, v2 - v0));
   }
-  for (int i = tid; i < T.nv; i += BS) {
+  for (int i = tid; i < nv; i += BS) {
     const D3 p = c.pos(i);
     q[2] += p.x;
     q[3] += p.y;
@@ -182,29 +198,32 @@ __global__ __launch_bounds__(BS) void k_cell_stats(VertexDev V, TypeDev T, const
     q[11] = fmax(q[11], p.y);
     q[12] = fmin(q[12], p.z);
     q[13] = fmax(q[13], p.z);
-    for (int j = i + 1; j < T.nv; ++j) {
-      const D3 r = c.pos(j);
-      const double dx = p.x - r.x, dy = p.y - r.y, dz = p.z - r.z;
-      q[14] = fmax(q[14], sqrt(dx * dx + dy * dy + dz * dz));
+    for (int k = 1; k <= nv / 2; ++k) {
+      const D3 o = c.pos(i + k < nv ? i + k : i + k - nv);
+      const double dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
+      q[14] = fmax(q[14], dx * dx + dy * dy + dz * dz);
     }
   }
-  for (int k = 0; k < NQ; ++k) red[k][tid] = q[k];
+  // over the wavefront, then over the wavefronts
+#pragma unroll
+  for (int k = 0; k < NQ; ++k) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const double y = __shfl_xor(q[k], o);
+      q[k] = k < 8 ? q[k] + y : (k < 14 && (k & 1) == 0 ? fmin(q[k], y) : fmax(q[k], y));
+    }
+    if ((tid & 63) == 0) red[k][tid >> 6] = q[k];
+  }
   __syncthreads();
-  for (int h = BS / 2; h > 0; h >>= 1) {
-    if (tid < h) {
-      for (int k = 0; k < 8; ++k) red[k][tid] += red[k][tid + h];
-      for (int k = 8; k < 14; k += 2) {
-        red[k][tid] = fmin(red[k][tid], red[k][tid + h]);
-        red[k + 1][tid] = fmax(red[k + 1][tid], red[k + 1][tid + h]);
-      }
-      red[14][tid] = fmax(red[14][tid], red[14][tid + h]);
-    }
-    __syncthreads();
-  }
   if (tid < NQ) {
-    double r = red[tid][0];
-    if (tid >= 2 && tid < 8) r /= (double)T.nv;
-    out[(int64_t)NQ * cell + tid] = r;
+    double v = red[tid][0];
+    for (int w = 1; w < NW; ++w) {
+      const double y = red[tid][w];
+      v = tid < 8 ? v + y : (tid < 14 && (tid & 1) == 0 ? fmin(v, y) : fmax(v, y));
+    }
+    if (tid >= 2 && tid < 8) v /= (double)nv;
+    if (tid == 14) v = sqrt(v);
+    out[(int64_t)NQ * cell + tid] = v;
   }
 }
 
@@ -268,7 +287,12 @@ hipError_t launch_mechanics(hipStream_t s, const VertexDev& V, const TypeDev& T,
 hipError_t launch_cell_stats(hipStream_t s, const VertexDev& V, const TypeDev& T, const int32_t* cells, int ncells,
                              const int64_t* cell_base, double* out) {
   if (ncells <= 0) return hipSuccess;
-  hipLaunchKernelGGL((k_cell_stats<128>), dim3((unsigned)ncells), dim3(128), 0, s, V, T, cells, cell_base, out);
+  const dim3 g((unsigned)ncells), b(256);
+  if (T.nv <= kStatsStaged)
+    hipLaunchKernelGGL((k_cell_stats<256, true>), g, b, sizeof(double) * 3 * (size_t)T.nv, s, V, T, cells, cell_base,
+                       out);
+  else
+    hipLaunchKernelGGL((k_cell_stats<256, false>), g, b, 0, s, V, T, cells, cell_base, out);
   return hipGetLastError();
 }
 
