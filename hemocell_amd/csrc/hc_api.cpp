@@ -510,7 +510,7 @@ hc_status build_dense_extra(hc_ctx* ctx) {
 }
 
 void free_repulsion(hc_ctx* ctx) {
-  void* ps[] = {ctx->rb.keys_in, ctx->rb.keys_out, ctx->rb.ids_in, ctx->rb.ids_out, ctx->rb.temp, ctx->d_vcell};
+  void* ps[] = {ctx->rb.keys, ctx->rb.ranks, ctx->rb.entries, ctx->rb.used, ctx->d_vcell};
   for (void* p : ps)
     if (p) hipFree(p);
   RepulsionBufs z{};
@@ -520,7 +520,7 @@ void free_repulsion(hc_ctx* ctx) {
   ctx->rb_nv = -1;
 }
 
-// Sort buffers sized for the current vertices, the cell index of every vertex,
+// Bin entries sized for the current vertices, the cell index of every vertex,
 // and the per-node bin bounds (zeroed once; the repulsion launch leaves them zero).
 hc_status ensure_repulsion(hc_ctx* ctx) {
   hc_status s;
@@ -532,11 +532,11 @@ hc_status ensure_repulsion(hc_ctx* ctx) {
   HC_TRY(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
   free_repulsion(ctx);
   const int64_t nv = std::max<int64_t>(ctx->nv, 1);
-  void** bufs[4] = {(void**)&ctx->rb.keys_in, (void**)&ctx->rb.keys_out, (void**)&ctx->rb.ids_in, (void**)&ctx->rb.ids_out};
-  for (void** b : bufs)
-    if ((s = dalloc(ctx, b, 4 * nv, "repulsion sort buffers")) != HC_OK) return s;
-  ctx->rb.temp_bytes = repulsion_temp_bytes(ctx->nv, ctx->L.N);
-  if ((s = dalloc(ctx, &ctx->rb.temp, std::max<size_t>(ctx->rb.temp_bytes, 16), "radix-sort scratch")) != HC_OK) return s;
+  if ((s = dalloc(ctx, (void**)&ctx->rb.keys, 4 * nv, "repulsion keys")) != HC_OK) return s;
+  if ((s = dalloc(ctx, (void**)&ctx->rb.ranks, 4 * nv, "repulsion ranks")) != HC_OK) return s;
+  if ((s = dalloc(ctx, (void**)&ctx->rb.entries, sizeof(BinEntry) * nv, "repulsion bin entries")) != HC_OK) return s;
+  if ((s = dalloc(ctx, (void**)&ctx->rb.used, 256, "repulsion entry count")) != HC_OK) return s;
+  HC_TRY(hipMemsetAsync(ctx->rb.used, 0, 256, ctx->stream), "hipMemsetAsync");
   std::vector<int32_t> vcell((size_t)nv, 0);
   for (size_t c = 0; c < ctx->cell_base.size(); ++c) {
     const int n = ctx->types[ctx->cell_type[c]]->host.nv;

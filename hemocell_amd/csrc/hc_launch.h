@@ -105,15 +105,18 @@ hipError_t launch_cell_step_mixed(hipStream_t s, const VertexDev& V, const TypeD
                                   int box_bytes, int lds_device, unsigned long long* wall_hits);
 
 // binning and cell-cell repulsion (hc_repulsion.hip)
-struct RepulsionBufs {
-  uint32_t *keys_in, *keys_out;  // nearest-node key per vertex, before / after the sort
-  int32_t *ids_in, *ids_out;     // vertex ids, sorted alongside
-  int2* bins;                    // [start, end) per node into ids_out; all zero between launches
-  const int32_t* vcell;          // cell index of each vertex
-  void* temp;                    // radix-sort scratch
-  size_t temp_bytes;
+struct BinEntry {  // one vertex in its bin
+  double x, y, z;
+  int32_t id, cell;
 };
-size_t repulsion_temp_bytes(int64_t nv, int64_t N);
+struct RepulsionBufs {
+  uint32_t* keys;        // nearest-node key per vertex
+  int32_t* ranks;        // its place of arrival among the vertices of that node
+  BinEntry* entries;     // the vertices by node, ascending ids within a node
+  int2* bins;            // [start, end) per node into entries; all zero between launches
+  int* used;             // entries in use; zero between launches
+  const int32_t* vcell;  // cell index of each vertex
+};
 hipError_t launch_repulsion(hipStream_t s, const VertexDev& V, const LatticeDev& L, const RepulsionBufs& B,
                             double k_rep, double r_c);
 // boundary particles (bounce-back nodes next to a non-bounce-back node) and the

@@ -271,7 +271,10 @@ hipError_t launch_mechanics(hipStream_t s, const VertexDev& V, const TypeDev& T,
       HC_MECH(HC_MODEL_RBC, 256)
       break;
     case HC_MODEL_PLT:
-      HC_MECH(HC_MODEL_PLT, 64)
+      // few platelets: their latency sets the time, and 66 vertices fit one round of
+      // two wavefronts (24 platelets 47 -> 30 us)
+      if (ncells < 256) { HC_MECH(HC_MODEL_PLT, 128) }
+      else { HC_MECH(HC_MODEL_PLT, 64) }
       break;
     case HC_MODEL_WBC:
       HC_MECH(HC_MODEL_WBC, 256)

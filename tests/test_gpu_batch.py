@@ -120,3 +120,4 @@ def test_empty_and_ragged_inputs():
     for pair in sims:
         for s in pair:
             s.close()
+
