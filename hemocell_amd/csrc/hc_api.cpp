@@ -685,7 +685,7 @@ int cell_threads(const hc_ctx* c, int model, bool few) {
 // every type in one persistent launch on the context stream; false when the
 // launch does not apply (no queue, or the layout does not fit the LDS)
 template <typename R>
-bool mixed_cell_step(hc_ctx* ctx, int do_interp, hc_status& st) {
+bool mixed_cell_step(hc_ctx* ctx, int do_interp, bool spread, hc_status& st) {
   st = HC_OK;
   if (!ctx->mixed || !ctx->d_queue || ctx->nqueue == 0) return false;
   std::vector<TypeDev> ht(ctx->types.size());
@@ -693,10 +693,9 @@ bool mixed_cell_step(hc_ctx* ctx, int do_interp, hc_status& st) {
   for (size_t t = 0; t < ht.size(); ++t) {
     const TypeBufs& tb = *ctx->types[t];
     ht[t] = tb.dev;
-    int f = CELL_FLAG_SPREAD;
+    int f = spread ? CELL_FLAG_SPREAD : 0;
     if (do_interp) f |= CELL_FLAG_INTERP;
     if ((ctx->iter % tb.host.timescale) == 0) f |= CELL_FLAG_MECH;
-    if (ctx->repulsion) f |= CELL_FLAG_REPULSION;
     flags[t] = f;
   }
   const int box = spread_box_bytes(ctx, HC_MODEL_RBC, false);
@@ -730,12 +729,12 @@ BoxCase box_case(hc_ctx* c, int cur) {
 }
 
 template <typename R>
-hc_status do_cell_step(hc_ctx* ctx, int do_interp) {
+hc_status do_cell_step(hc_ctx* ctx, int do_interp, bool spread) {
   hipEvent_t ev;
   prof_begin(ctx, HC_PROF_MECH, &ev);
   {
     hc_status st;
-    if (mixed_cell_step<R>(ctx, do_interp, st)) {
+    if (mixed_cell_step<R>(ctx, do_interp, spread, st)) {
       prof_end(ctx, HC_PROF_MECH, ev);
       return st;
     }
@@ -760,10 +759,9 @@ hc_status do_cell_step(hc_ctx* ctx, int do_interp) {
     const size_t k = (kk + 1) % act.size();
     TypeBufs& tb = *act[k];
     hipStream_t st = (k == 0 || nside == 0) ? ctx->stream : ctx->side[(k - 1) % nside];
-    int flags = CELL_FLAG_SPREAD;
+    int flags = spread ? CELL_FLAG_SPREAD : 0;
     if (do_interp) flags |= CELL_FLAG_INTERP;
     if ((ctx->iter % tb.host.timescale) == 0) flags |= CELL_FLAG_MECH;
-    if (ctx->repulsion) flags |= CELL_FLAG_REPULSION;
     const bool few = tb.ncells < ctx->n_cu;
     int block = cell_threads(ctx, tb.host.model, few);
     // while compute units are left over beside the main type, a large side cell
@@ -896,7 +894,11 @@ hc_status one_step(hc_ctx* ctx) {
   hipEvent_t ev;
   prof_begin(ctx, HC_PROF_STEP, &ev);
   const bool iv = iv_active(ctx) && ctx->nv > 0;
-  const bool fused = ctx->fuse && !ctx->repulsion && !ctx->brep && ctx->nv > 0;
+  // The repulsion of the next step comes before its spread, which the cell kernel
+  // then leaves out.  FP32 keeps the separate passes there: their mechanics are in
+  // FP64, the cell kernel's are not.
+  const bool ahead = !ctx->repulsion && !ctx->brep;
+  const bool fused = ctx->fuse && ctx->nv > 0 && (ahead || std::is_same<R, double>::value);
   // interior viscosity (hemoCell.cpp:347-357): after the constitutive model; the
   // membrane pass takes the support of the positions before the advance
   const bool memb = iv && ctx->iter % ctx->iv_timescale == 0;
@@ -927,7 +929,7 @@ hc_status one_step(hc_ctx* ctx) {
                "velocity_field");
       prof_end(ctx, HC_PROF_INTERP, e2);
     }
-    if ((s = do_cell_step<R>(ctx, do_interp)) != HC_OK) return s;
+    if ((s = do_cell_step<R>(ctx, do_interp, ahead)) != HC_OK) return s;
   } else {
     if ((s = do_interp_advance<R>(ctx, do_interp, 1)) != HC_OK) return s;
     if ((s = do_mechanics(ctx, false)) != HC_OK) return s;
@@ -935,7 +937,7 @@ hc_status one_step(hc_ctx* ctx) {
   if (grid && (s = do_visc_grid(ctx)) != HC_OK) return s;
   if (memb && (s = do_visc_membrane(ctx, ctx->d_xold)) != HC_OK) return s;
   if ((s = do_end<R>(ctx)) != HC_OK) return s;
-  ctx->spread_ready = fused;
+  ctx->spread_ready = fused && ahead;
   prof_end(ctx, HC_PROF_STEP, ev);
   if (ctx->prof.on && ctx->prof.used > 4096) prof_flush(ctx);
   return HC_OK;

@@ -31,7 +31,7 @@
 namespace hcg {
 namespace {
 
-enum { CELL_INTERP = 1, CELL_MECH = 2, CELL_SPREAD = 4, CELL_REPULSION = 8 };
+enum { CELL_INTERP = 1, CELL_MECH = 2, CELL_SPREAD = 4 };
 // 64-triangle chunks of a mesh whose volume is summed in an order independent of
 // the block size (meshes up to 8192 triangles)
 constexpr int kVolChunks = 128;
@@ -367,6 +367,16 @@ __device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev
         bz[k] = b.z;
       }
     }
+    // A platelet's edges once each, for the vertices to gather: by vertex, every
+    // edge was evaluated four times and a vertex's twelve one after another
+    // (24 platelets in FP64: this kernel 51 -> 37 us).
+    P* edge_f = nullptr;
+    if constexpr (MODEL == HC_MODEL_PLT && STAGED) {
+      if (6 * (size_t)T.ne * sizeof(P) <= platelet_edge_bytes(nv, sizeof(P))) {
+        edge_f = reinterpret_cast<P*>(region);
+        for (int e = tid; e < T.ne; e += BS) platelet_edge(c, T, e, vx, vy, vz, edge_f + e, T.ne);
+      }
+    }
     __syncthreads();
     const P vforce = (P)vforce_sh;
     for (int k = tid; k < nv; k += BS) {
@@ -375,7 +385,7 @@ __device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev
         F = T.rpar ? vertex_force_rbc_r(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc)
             : compact ? vertex_force_rbc_c(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc)
                       : vertex_force<MODEL, TERM_ALL, P>(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc);
-      else F = vertex_force<MODEL, TERM_ALL, P>(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc);
+      else F = vertex_force<MODEL, TERM_ALL, P>(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc, edge_f);
       const int64_t i = base + k;
       double f0 = (double)F.x, f1 = (double)F.y, f2 = (double)F.z;
       if (flags & CELL_SPREAD) cap_force(i, f0, f1, f2);
@@ -391,8 +401,8 @@ __device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev
   // the force each vertex spreads: its force plus any extra force, capped to
   // f_limit and written back in place when that changed it
   // (hemoCellParticleField.cpp:846-852; done by the mechanics above when it ran
-  // on this cell), plus the repulsion force when enabled.  The packed positions
-  // below overwrite the offsets: the mechanics ended with a barrier.
+  // on this cell); with repulsion the spread is a pass of its own.  The packed
+  // positions below overwrite the offsets: the mechanics ended with a barrier.
   {
     int lmin[3] = {0x7fffffff, 0x7fffffff, 0x7fffffff}, lmax[3] = {-0x7fffffff, -0x7fffffff, -0x7fffffff};
     bool lbad = false, lfar = false;
@@ -458,11 +468,6 @@ __device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev
     f0 = V.f[i];
     f1 = V.f[vs + i];
     f2 = V.f[2 * vs + i];
-    if (flags & CELL_REPULSION) {
-      f0 = V.frep[i] + f0;
-      f1 = V.frep[vs + i] + f1;
-      f2 = V.frep[2 * vs + i] + f2;
-    }
   };
   if (direct) {
     for (int k = tid; k < nv; k += BS) {

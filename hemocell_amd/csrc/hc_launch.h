@@ -82,7 +82,7 @@ hipError_t launch_interleave(hipStream_t s, const double* const* src, int nf, in
                              double* out);
 
 // fused per-cell step (hc_cell_body.h): interpolation + advance, mechanics, next spread
-enum { CELL_FLAG_INTERP = 1, CELL_FLAG_MECH = 2, CELL_FLAG_SPREAD = 4, CELL_FLAG_REPULSION = 8 };
+enum { CELL_FLAG_INTERP = 1, CELL_FLAG_MECH = 2, CELL_FLAG_SPREAD = 4 };
 template <typename R>
 hipError_t launch_cell_step(hipStream_t s, const VertexDev& V, const TypeDev& T, const int32_t* cells, int ncells,
                             const int64_t* cell_base, const R* uf, const uint8_t* type, const LatticeDev& L,

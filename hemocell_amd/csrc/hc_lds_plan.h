@@ -6,8 +6,9 @@
 //   fixed   positions (3 nv scalars) and, staged with a viscous membrane, the
 //           vertex velocities (3 nv more), rounded up to 16 bytes; in the plain
 //           layout 3 nv doubles; nothing when the positions stay in global memory;
-//   region  the bending forces of the mechanics (staged, 3 nv scalars) and then
-//           the spread box (3 doubles per node) over the same bytes;
+//   region  the bending forces of the mechanics (staged, 3 nv scalars; platelets:
+//           the terms of each edge, 6 scalars) and then the spread box (3 doubles
+//           per node) over the same bytes;
 //   lists   the spread's bucketed vertex list (2 bytes per vertex), which the
 //           kernel places right after the box's last node.
 #pragma once
@@ -24,6 +25,17 @@ constexpr size_t cell_fixed_bytes(int nv, bool visc, size_t psize, bool staged, 
   return gpos ? 0 : (staged ? (((visc ? 6 : 3) * (size_t)nv * psize + 15) & ~(size_t)15) : 3 * (size_t)nv * sizeof(double));
 }
 
+// the terms of a platelet's edges, of which a closed surface has fewer than 3 nv;
+// 0 for a mesh whose edges are evaluated by each of their vertices instead
+constexpr size_t platelet_edge_bytes(int nv, size_t psize) {
+  return 18 * (size_t)nv * psize <= 32768 ? 18 * (size_t)nv * psize : 0;
+}
+
+// what the staged mechanics keeps in the region
+constexpr size_t cell_mech_bytes(int model, int nv, size_t psize) {
+  return model == LDS_MODEL_PLT ? platelet_edge_bytes(nv, psize) : 3 * (size_t)nv * psize;
+}
+
 constexpr size_t cell_list_bytes(int nv) { return (2 * (size_t)nv + 15) & ~(size_t)15; }
 
 struct CellLdsPlan {
@@ -35,16 +47,16 @@ struct CellLdsPlan {
 
 // One cell type's layout for a launch of the per-type kernel.  st_* are the
 // static LDS bytes of the staged, plain and global-position instantiations.
-// Staged when positions, velocities, bending forces and the box fit; otherwise
+// Staged when positions, velocities, the mechanics' region and the box fit; otherwise
 // positions plus as much box as fits; with gpos only the box.
 inline CellLdsPlan cell_lds_plan(int model, int nv, bool visc, size_t psize, size_t box_bytes, size_t lds_device,
                                  size_t st_staged, size_t st_plain, size_t st_gpos, bool gpos) {
   CellLdsPlan p{};
-  const size_t bend = model != LDS_MODEL_PLT ? 3 * (size_t)nv * psize : 0;
+  const size_t mech = cell_mech_bytes(model, nv, psize);
   p.lists = cell_list_bytes(nv);
   p.staged = !gpos;
   p.fixed = cell_fixed_bytes(nv, visc, psize, p.staged, gpos);
-  p.region = p.staged ? std::max(bend, box_bytes) : box_bytes;
+  p.region = p.staged ? std::max(mech, box_bytes) : box_bytes;
   if (p.staged && p.fixed + p.region + p.lists + st_staged + kLdsMargin > lds_device) {
     p.staged = false;
     p.fixed = cell_fixed_bytes(nv, visc, sizeof(double), false, false);
@@ -67,9 +79,9 @@ inline size_t mixed_lds_plan(int ntypes, const int* model, const int* nv, const 
   size_t dyn = 0;
   for (int t = 0; t < ntypes; ++t) {
     const bool gpos = model[t] == LDS_MODEL_WBC;
-    const size_t bend = (!gpos && model[t] != LDS_MODEL_PLT) ? 3 * (size_t)nv[t] * psize : 0;
+    const size_t mech = gpos ? 0 : cell_mech_bytes(model[t], nv[t], psize);
     const size_t fixed = cell_fixed_bytes(nv[t], visc[t], psize, !gpos, gpos);
-    dyn = std::max(dyn, fixed + std::max(bend, box_bytes) + cell_list_bytes(nv[t]));
+    dyn = std::max(dyn, fixed + std::max(mech, box_bytes) + cell_list_bytes(nv[t]));
   }
   dyn = (dyn + 15) & ~(size_t)15;
   if (dyn + st + kLdsMargin > lds_device) return 0;

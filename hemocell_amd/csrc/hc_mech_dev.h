@@ -153,14 +153,56 @@ __device__ V3T<M> bending_force(const CellViewT<M>& c, const TypeDev& T, int i) 
 enum { TERM_AREA = 1, TERM_VOLUME = 2, TERM_BENDING = 4, TERM_LINK = 8, TERM_VISC = 16, TERM_INNER = 32,
        TERM_ALL = 63 };
 
+// Link and membrane viscosity force of a platelet's edge on its first vertex (the
+// second takes the opposite) and its dihedral bending force (on both, and with the
+// opposite sign on the two vertices across), the terms and operations of
+// vertex_force below.  out: 6 scalars, stride apart.
+template <typename M>
+__device__ __forceinline__ void platelet_edge(const CellViewT<M>& c, const TypeDev& T, int ed, const M* vx, const M* vy,
+                                              const M* vz, M* out, int stride) {
+  const int a = T.edge[2 * ed], b = T.edge[2 * ed + 1];
+  const int32_t* T0 = T.tri + 3 * T.edge_tris[2 * ed];
+  const int32_t* T1 = T.tri + 3 * T.edge_tris[2 * ed + 1];
+  const M l0 = (M)T.edge_len_eq[ed], angle_eq = (M)T.edge_angle_eq[ed];
+  const V3T<M> ev = c.pos(b) - c.pos(a);
+  const M len = normp(ev);
+  const M il = mrcp(len);
+  const V3T<M> uv = {ev.x * il, ev.y * il, ev.z * il};
+  const M ef = mdiv(len - l0, l0);
+  const M fs = (M)T.k_link * (ef + mdiv(ef, mabs(M(MaxCellPersistenceLength) - ef * ef)));
+  const V3T<M> rv = {vx[b] - vx[a], vy[b] - vy[a], vz[b] - vz[a]};
+  const M pr = dotp(rv, uv);
+  const M eta = (M)T.eta_m;
+  V3T<M> fv = {(pr * uv.x) * eta, (pr * uv.y) * eta, (pr * uv.z) * eta};
+  const M m = normp(fv);
+  if (m > M(FORCE_LIMIT / 4.0)) {
+    const M s = mdiv(M(FORCE_LIMIT / 4.0), m);
+    fv.x *= s;
+    fv.y *= s;
+    fv.z *= s;
+  }
+  out[0] = uv.x * fs + fv.x;
+  out[stride] = uv.y * fs + fv.y;
+  out[2 * stride] = uv.z * fs + fv.z;
+  const V3T<M> n1 = unit_normal(c.pos(T0[0]), c.pos(T0[1]), c.pos(T0[2]));
+  const V3T<M> n2 = unit_normal(c.pos(T1[0]), c.pos(T1[1]), c.pos(T1[2]));
+  const M ang = matan2(dotp(crossp(n1, n2), uv), dotp(n1, n2));
+  const M af = ang - angle_eq;
+  const M fm = (M)T.k_bend * (af + mdiv(af, mabs(M(MaxPLTBendingAngle) - af * af)));
+  out[3 * stride] = ((n1.x + n2.x) * fm) * M(0.5);
+  out[4 * stride] = ((n1.y + n2.y) * fm) * M(0.5);
+  out[5 * stride] = ((n1.z + n2.z) * fm) * M(0.5);
+}
+
 // Force on vertex k of one cell: every term gathered in the reference's order
 // (area, volume, bending, edges, inner links), or only the terms in TERMS.
 // bx/by/bz: per-vertex bending forces of the cell; vx/vy/vz: vertex velocities
-// (membrane viscosity).
+// (membrane viscosity).  edge_f: a platelet's edge forces from platelet_edge (null:
+// each vertex evaluates its edges itself).
 template <int MODEL, int TERMS = TERM_ALL, typename M = double>
 __device__ __forceinline__ V3T<M> vertex_force(const CellViewT<M>& c, const TypeDev& T, int k, M vforce,
                                                const M* bx, const M* by, const M* bz, const M* vx, const M* vy,
-                                               const M* vz, bool visc) {
+                                               const M* vz, bool visc, const M* edge_f = nullptr) {
   M F0 = M(0), F1 = M(0), F2 = M(0);
   const V3T<M> xk = c.pos(k);
   // area and volume terms, triangle order: each incident triangle is evaluated
@@ -303,7 +345,24 @@ __device__ __forceinline__ V3T<M> vertex_force(const CellViewT<M>& c, const Type
       else { F0 -= bf.x; F1 -= bf.y; F2 -= bf.z; }
     }
   };
-  if (MODEL != HC_MODEL_PLT && T.vedge4p) {
+  if (MODEL == HC_MODEL_PLT && edge_f) {
+    const int S = T.ne;
+#pragma unroll 4
+    for (int e = T.vedge_off[k]; e < T.vedge_off[k + 1]; ++e) {
+      const int x = T.vedge4[e].x, kind = x & 3;
+      const M* const f = edge_f + (x >> 2);
+      if (kind != 2) {
+        const M sgn = kind == 0 ? M(1) : M(-1);
+        F0 = F0 + sgn * f[0] + f[3 * S];
+        F1 = F1 + sgn * f[S] + f[4 * S];
+        F2 = F2 + sgn * f[2 * S] + f[5 * S];
+      } else {
+        F0 -= f[3 * S];
+        F1 -= f[4 * S];
+        F2 -= f[5 * S];
+      }
+    }
+  } else if (MODEL != HC_MODEL_PLT && T.vedge4p) {
     int4 q[kPadW];
     M l0[kPadW];
 #pragma unroll
