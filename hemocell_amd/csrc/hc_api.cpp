@@ -62,6 +62,7 @@ struct hc_ctx {
   double tau = 1.0;
   void* f = nullptr;
   void* Fibm[2] = {nullptr, nullptr};
+  int64_t wall_nodes = 0;  // nodes that are not fluid
   void* ufield = nullptr;  // fluid velocity per node, filled before the interpolation
   uint8_t* type = nullptr;
   uint32_t* vel_nodes = nullptr;  // nodes with a velocity boundary
@@ -728,6 +729,11 @@ BoxCase box_case(hc_ctx* c, int cur) {
   return b;
 }
 
+// The node types for the velocity pass over all nodes, which then leaves the walls
+// out: with a tenth of them or more (a tube's corners are a fifth); a channel's two
+// planes of 512 do not pay for the types read.
+const uint8_t* walled(const hc_ctx* ctx) { return 10 * ctx->wall_nodes >= ctx->L.N ? ctx->type : nullptr; }
+
 template <typename R>
 hc_status do_cell_step(hc_ctx* ctx, int do_interp, bool spread) {
   hipEvent_t ev;
@@ -815,7 +821,7 @@ hc_status do_collide(hc_ctx* ctx) {
   prof_begin(ctx, HC_PROF_COLLIDE, &ev);
   HC_TRY(launch_collide_stream<R>(ctx->stream, (R*)ctx->f, (const R*)ctx->Fibm[ctx->cur], (R*)ctx->Fibm[1 - ctx->cur],
                                   ctx->type, ctx->L, a, ctx->phase, ctx->general, ctx->vel_nodes, ctx->n_vel,
-                                  ctx->fuse_vel),
+                                  ctx->fuse_vel, ctx->nv > 0),
          "collide_stream");
   prof_end(ctx, HC_PROF_COLLIDE, ev);
   ctx->phase ^= 1;
@@ -852,7 +858,7 @@ hc_status do_interp_advance(hc_ctx* ctx, int do_interp, int do_advance) {
   prof_begin(ctx, HC_PROF_INTERP, &ev);
   if (do_interp)
     HC_TRY(launch_velocity_field<R>(ctx->stream, (const R*)ctx->f, (const R*)ctx->Fibm[ctx->cur], (R*)ctx->ufield,
-                                    ctx->L, ctx->phase, ctx->general, ctx->g),
+                                    walled(ctx), ctx->L, ctx->phase, ctx->general, ctx->g),
            "velocity_field");
   HC_TRY(launch_interp_advance<R>(ctx->stream, vdev(ctx), (const R*)ctx->ufield, ctx->type, ctx->L, do_interp,
                                   do_advance, ctx->d_wall_hits),
@@ -925,7 +931,7 @@ hc_status one_step(hc_ctx* ctx) {
                "velocity_field");
       else
         HC_TRY(launch_velocity_field<R>(ctx->stream, (const R*)ctx->f, (const R*)ctx->Fibm[ctx->cur], (R*)ctx->ufield,
-                                        ctx->L, ctx->phase, ctx->general, ctx->g),
+                                        walled(ctx), ctx->L, ctx->phase, ctx->general, ctx->g),
                "velocity_field");
       prof_end(ctx, HC_PROF_INTERP, e2);
     }
@@ -1619,13 +1625,13 @@ hc_status hc_lattice_init(hc_ctx* ctx, int nx, int ny, int nz, const uint8_t* no
   ctx->L.N = N;
   ctx->L.stride = (N + 255) / 256 * 256;
   ctx->L.spread_q = ctx->L.spread_inv_q = 0.0;  // plain adds until hc_set_exact_spread
-  bool has_walls = false;
+  int64_t walls = 0;
   std::vector<uint32_t> vel;
   if (node_type) {
     for (int64_t n = 0; n < N; ++n) {
       uint8_t t = node_type[n];
       if (t > HC_NODE_VELOCITY + 5) return fail(ctx, HC_INVALID_ARG, "unknown node type in mask");
-      if (t != HC_NODE_FLUID) has_walls = true;
+      if (t != HC_NODE_FLUID) ++walls;
       if (t >= HC_NODE_VELOCITY) {
         // a velocity node must sit on the domain face it names
         const int face = t - HC_NODE_VELOCITY, axis = face >> 1;
@@ -1640,7 +1646,9 @@ hc_status hc_lattice_init(hc_ctx* ctx, int nx, int ny, int nz, const uint8_t* no
   }
   // grouped by face, so that the lanes of a wavefront take the same face branch
   std::stable_sort(vel.begin(), vel.end(), [&](uint32_t a, uint32_t b) { return node_type[a] < node_type[b]; });
+  const bool has_walls = walls > 0;
   ctx->has_walls = has_walls;
+  ctx->wall_nodes = walls;
   ctx->general = has_walls || !all_periodic;
   const size_t rs = rsize(ctx);
   hc_status s;

@@ -80,6 +80,9 @@ __device__ __forceinline__ NbrOff neighbour_offsets(int x, int y, int z, const L
   o.zp = z < L.nz - 1 ? 1 : (L.periodic[2] ? -(L.nz - 1) : INVALID);
   return o;
 }
+__device__ __forceinline__ bool closed_face(const NbrOff& o) {
+  return o.xm == INVALID || o.xp == INVALID || o.ym == INVALID || o.yp == INVALID || o.zm == INVALID || o.zp == INVALID;
+}
 // offset of node n + (DX, DY, DZ); sets ok = false when it leaves the domain
 template <int DX, int DY, int DZ, bool CHECK>
 __device__ __forceinline__ int nbr_offset(const NbrOff& o, bool& ok) {

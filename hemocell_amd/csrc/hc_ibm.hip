@@ -114,11 +114,14 @@ __device__ __forceinline__ void velocity_node_field(const R* __restrict__ f, con
   q[2] = j2 * invRho + (R(g2) + Fcur[2 * S + n]) / R(2);
 }
 
-template <typename R, bool PHASE1, bool CHECK>
+// WALLS: nodes that are not fluid are left out; no support gives them a weight.
+template <typename R, bool PHASE1, bool CHECK, bool WALLS>
 __global__ __launch_bounds__(BLOCK) void k_velocity_field(const R* __restrict__ f, const R* __restrict__ Fcur,
-                                                          R* __restrict__ uf, LatticeDev L, double g0, double g1,
-                                                          double g2) {
-  velocity_node_field<R, PHASE1, CHECK>(f, Fcur, uf, L, g0, g1, g2, blockIdx.x * BLOCK + threadIdx.x);
+                                                          R* __restrict__ uf, const uint8_t* __restrict__ type,
+                                                          LatticeDev L, double g0, double g1, double g2) {
+  const uint32_t n = blockIdx.x * BLOCK + threadIdx.x;
+  if (WALLS && n < (uint32_t)L.N && type[n] != HC_NODE_FLUID) return;
+  velocity_node_field<R, PHASE1, CHECK>(f, Fcur, uf, L, g0, g1, g2, n);
 }
 
 // several independent lattices in one launch; case c owns the blocks from c.block0
@@ -417,15 +420,24 @@ hipError_t launch_spread_cells(hipStream_t s, const VertexDev& V, R* Fibm, const
 }
 
 template <typename R>
-hipError_t launch_velocity_field(hipStream_t s, const R* f, const R* Fcur, R* uf, const LatticeDev& L, int phase,
-                                 bool general, const double g[3]) {
+hipError_t launch_velocity_field(hipStream_t s, const R* f, const R* Fcur, R* uf, const uint8_t* type,
+                                 const LatticeDev& L, int phase, bool general, const double g[3]) {
   dim3 gr = grid_for(L.N);
-  if (phase) {
-    if (general) hipLaunchKernelGGL((k_velocity_field<R, true, true>), gr, dim3(BLOCK), 0, s, f, Fcur, uf, L, g[0], g[1], g[2]);
-    else hipLaunchKernelGGL((k_velocity_field<R, true, false>), gr, dim3(BLOCK), 0, s, f, Fcur, uf, L, g[0], g[1], g[2]);
+#define HC_VELOCITY(PHASE1, CHECK)                                                                               \
+  if (type)                                                                                                      \
+    hipLaunchKernelGGL((k_velocity_field<R, PHASE1, CHECK, true>), gr, dim3(BLOCK), 0, s, f, Fcur, uf, type, L, g[0], \
+                       g[1], g[2]);                                                                              \
+  else                                                                                                           \
+    hipLaunchKernelGGL((k_velocity_field<R, PHASE1, CHECK, false>), gr, dim3(BLOCK), 0, s, f, Fcur, uf, type, L, g[0], \
+                       g[1], g[2])
+  if (phase && general) {
+    HC_VELOCITY(true, true);
+  } else if (phase) {
+    HC_VELOCITY(true, false);
   } else {
-    hipLaunchKernelGGL((k_velocity_field<R, false, false>), gr, dim3(BLOCK), 0, s, f, Fcur, uf, L, g[0], g[1], g[2]);
+    HC_VELOCITY(false, false);
   }
+#undef HC_VELOCITY
   return hipGetLastError();
 }
 
@@ -498,8 +510,8 @@ hipError_t launch_interleave(hipStream_t s, const double* const* src, int nf, in
                                        int);                                                                         \
   template hipError_t launch_spread_cells<R>(hipStream_t, const VertexDev&, R*, const uint8_t*, const LatticeDev&,    \
                                              const int64_t*, const int32_t*, int, double, int, int);                  \
-  template hipError_t launch_velocity_field<R>(hipStream_t, const R*, const R*, R*, const LatticeDev&, int, bool,     \
-                                               const double*);                                                       \
+  template hipError_t launch_velocity_field<R>(hipStream_t, const R*, const R*, R*, const uint8_t*, const LatticeDev&, \
+                                               int, bool, const double*);                                                       \
   template hipError_t launch_velocity_boxes<R>(hipStream_t, const BoxCase&, int, int, bool);                          \
   template hipError_t launch_velocity_boxes_multi<R>(hipStream_t, const BoxCase*, int, int, bool);                    \
   template hipError_t launch_interp_advance<R>(hipStream_t, const VertexDev&, const R*, const uint8_t*,               \

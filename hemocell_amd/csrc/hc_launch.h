@@ -19,7 +19,7 @@ struct CollideArgs {
 template <typename R>
 hipError_t launch_collide_stream(hipStream_t s, R* f, const R* Fcur, R* Fclear, const uint8_t* type,
                                  const LatticeDev& L, const CollideArgs& a, int odd, bool general,
-                                 const uint32_t* vel_nodes, int n_vel, bool fuse_vel);
+                                 const uint32_t* vel_nodes, int n_vel, bool fuse_vel, bool force);
 template <typename R>
 hipError_t launch_init_equilibrium(hipStream_t s, R* f, const uint8_t* type, const LatticeDev& L,
                                    double rho, const double u[3]);
@@ -70,8 +70,8 @@ hipError_t launch_spread_cells(hipStream_t s, const VertexDev& V, R* Fibm, const
                                const int64_t* cell_base, const int32_t* cell_nv, int ncells, double f_limit,
                                int use_repulsion, int lds_bytes);
 template <typename R>
-hipError_t launch_velocity_field(hipStream_t s, const R* f, const R* Fcur, R* uf, const LatticeDev& L, int phase,
-                                 bool general, const double g[3]);
+hipError_t launch_velocity_field(hipStream_t s, const R* f, const R* Fcur, R* uf, const uint8_t* type,
+                                 const LatticeDev& L, int phase, bool general, const double g[3]);
 template <typename R>
 hipError_t launch_interp_advance(hipStream_t s, const VertexDev& V, const R* uf, const uint8_t* type,
                                  const LatticeDev& L, int do_interp, int do_advance, unsigned long long* wall_hits);
