@@ -1810,11 +1810,17 @@ hc_status hc_add_cell_type(hc_ctx* ctx, int model, int nv, int nt, const int32_t
     D.cbend = nullptr;
     D.rpar = nullptr;
     D.rnb = nullptr;
+    D.rid = nullptr;
     if (!T.rpar.empty() && !padded_off(ctx) && !ring_tables_off()) {
       const float* pf = nullptr;
       if ((s = upload(ctx, *tb, T.rpar, &pf)) != HC_OK) return s;
       D.rpar = (const float4*)pf;
       if ((s = upload(ctx, *tb, T.rnb, &D.rnb)) != HC_OK) return s;
+      if (!T.rid.empty()) {
+        const uint32_t* pi = nullptr;
+        if ((s = upload(ctx, *tb, T.rid, &pi)) != HC_OK) return s;
+        D.rid = (const uint4*)pi;
+      }
     }
     if (!T.cslot.empty() && !padded_off(ctx)) {
       const uint32_t* pc = nullptr;

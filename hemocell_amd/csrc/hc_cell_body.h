@@ -322,76 +322,149 @@ __device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev
     }
     __syncthreads();
   } else if (flags & CELL_MECH) {
+    // FP64: roots and quotients once per triangle and edge (hc_mech_dev.h).  Region
+    // left beside the bending forces for both lists of factors: everything is
+    // evaluated at once, then gathered; otherwise one after the other, with the
+    // vertices' sums in V.f between.  The sums are the same either way.  One
+    // RBC 57 -> 52 us per step; 120 x 136 x 250 nodes with 1886 RBC 765 -> 743.
+    constexpr bool kOnce = MODEL != HC_MODEL_PLT && STAGED && std::is_same<P, double>::value;
+    const bool once = kOnce && T.rid;  // at most 2 nv triangles and 3 nv edges
+    const bool apart = 3 * nv + T.nt + T.ne <= 3 * box_nodes;
+    P* const tri_f = reinterpret_cast<P*>(region) + (apart ? 3 * nv : 0);
     // the volume: triangle t is lane t % 64 of chunk t / 64; a wavefront sums a
-    // chunk by a butterfly over its lanes and thread 0 adds the chunks in order,
-    // so the sum is the same at every block size (batched, mixed and alone
-    // launches agree bit for bit); larger meshes sum per thread, then per
-    // wavefront
+    // chunk over its lanes (by moves between registers: through LDS the six steps
+    // cost a fifth of the mechanics) and the chunks are added in order, so the sum
+    // is the same at every block size (batched, mixed and alone launches agree bit
+    // for bit); larger meshes sum per thread, then per wavefront
     const int nchunk = (T.nt + 63) >> 6;
     int nred = nchunk;
     if (nchunk <= kVolChunks) {
       const V3T<P> rm = c.pos(0);
       const D3 r = {(double)rm.x, (double)rm.y, (double)rm.z};
       for (int ch = tid >> 6; ch < nchunk; ch += BS / 64) {
-        double part = volume_term(c, T, (ch << 6) | (tid & 63), r);
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o);
-        if ((tid & 63) == 0) red[ch] = part;
+        const int t = (ch << 6) | (tid & 63);
+        const double part = wave_sum63(volume_term(c, T, t, r));
+        if ((tid & 63) == 63) red[ch] = part;
+        if (kOnce && once && t < T.nt) tri_f[t] = triangle_factor(c, T, t);
       }
     } else {
-      double part = volume_partial<BS>(c, T, tid);
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o);
-      if ((tid & 63) == 0) red[tid >> 6] = part;
+      const double part = wave_sum63(volume_partial<BS>(c, T, tid));
+      if ((tid & 63) == 63) red[tid >> 6] = part;
       nred = BS / 64;
+      if (kOnce && once)
+        for (int t = tid; t < T.nt; t += BS) tri_f[t] = triangle_factor(c, T, t);
     }
-    __syncthreads();
-    if (tid == 0) {
+    auto volume_force = [&]() {
       double vsum = red[0];
       for (int w = 1; w < nred; ++w) vsum += red[w];
       const double volume = vsum * (1.0 / 6.0);
       const double vf = (volume - T.volume_eq) / T.volume_eq;
-      vforce_sh = -T.k_volume * vf / fabs(MaxCellVolumetricChange - vf * vf);
+      return -T.k_volume * vf / fabs(MaxCellVolumetricChange - vf * vf);
+    };
+    if constexpr (kOnce) {
+      if (once) {
+        P* const edge_f = reinterpret_cast<P*>(region) + (apart ? 3 * nv + T.nt : 0);
+        auto edges = [&]() {
+          for (int e = tid; e < T.ne; e += BS) edge_f[e] = edge_factor(c, T, e, vx, vy, vz, visc);
+        };
+        auto bending = [&]() {
+          for (int k = tid; k < nv; k += BS) {
+            const RingOf ring(T, k);
+            const V3T<P> b = bending_of_ring<P>(c, T, k, ring.R, ring.nr);
+            bx[k] = b.x;
+            by[k] = b.y;
+            bz[k] = b.z;
+          }
+        };
+        // each of steps 1 (triangles), 2 (bending) and 4 (edges, inner links, cap)
+        // adds to the vertices' sums
+        auto gather = [&](int steps, P vforce) {
+          for (int k = tid; k < nv; k += BS) {
+            const int64_t i = base + k;
+            const RingOf ring(T, k);
+            P f0 = P(0), f1 = P(0), f2 = P(0);
+            if (steps & 1) {
+              gather_triangles<P>(c, T, ring, k, tri_f, vforce, f0, f1, f2);
+            } else {
+              f0 = V.f[i];
+              f1 = V.f[vs + i];
+              f2 = V.f[2 * vs + i];
+            }
+            if (steps & 2) gather_bending<P>(ring, k, bx, by, bz, f0, f1, f2);
+            if (steps & 4) {
+              gather_edges<P>(c, T, ring, k, edge_f, f0, f1, f2);
+              inner_forces<MODEL, P>(c, T, k, f0, f1, f2);
+              if (flags & CELL_SPREAD) cap_force(i, f0, f1, f2);
+            }
+            V.f[i] = f0;
+            V.f[vs + i] = f1;
+            V.f[2 * vs + i] = f2;
+          }
+        };
+        if (apart) {
+          bending();
+          edges();
+        }
+        __syncthreads();  // the factors, and the volume's partial sums
+        const P vforce = (P)volume_force();
+        if (apart) {
+          gather(7, vforce);
+        } else {
+          gather(1, vforce);
+          __syncthreads();
+          bending();
+          __syncthreads();
+          gather(2, P(0));
+          __syncthreads();
+          edges();
+          __syncthreads();
+          gather(4, P(0));
+        }
+      }
     }
-    // FP32 RBC: the ring-ordered tables, else the compact per-slot ones (both
-    // built beside the padded tables)
-    constexpr bool kCompact = MODEL == HC_MODEL_RBC && std::is_same<P, float>::value;
-    const bool compact = kCompact && T.cslot != nullptr;
-    if (MODEL != HC_MODEL_PLT) {
+    if (!once) {
+      __syncthreads();
+      if (tid == 0) vforce_sh = volume_force();
+      // FP32 RBC: the ring-ordered tables, else the compact per-slot ones (both
+      // built beside the padded tables)
+      constexpr bool kCompact = MODEL == HC_MODEL_RBC && std::is_same<P, float>::value;
+      const bool compact = kCompact && T.cslot != nullptr;
+      if (MODEL != HC_MODEL_PLT) {
+        for (int k = tid; k < nv; k += BS) {
+          V3T<P> b;
+          if constexpr (kCompact) b = compact ? bending_force_c(c, T, k) : bending_force(c, T, k);
+          else b = bending_force(c, T, k);
+          bx[k] = b.x;
+          by[k] = b.y;
+          bz[k] = b.z;
+        }
+      }
+      // A platelet's edges once each, for the vertices to gather: by vertex, every
+      // edge was evaluated four times and a vertex's twelve one after another
+      // (24 platelets in FP64: this kernel 51 -> 37 us).
+      P* edge_f = nullptr;
+      if constexpr (MODEL == HC_MODEL_PLT && STAGED) {
+        if (6 * (size_t)T.ne * sizeof(P) <= platelet_edge_bytes(nv, sizeof(P))) {
+          edge_f = reinterpret_cast<P*>(region);
+          for (int e = tid; e < T.ne; e += BS) platelet_edge(c, T, e, vx, vy, vz, edge_f + e, T.ne);
+        }
+      }
+      __syncthreads();
+      const P vforce = (P)vforce_sh;
       for (int k = tid; k < nv; k += BS) {
-        V3T<P> b;
-        if constexpr (kCompact) b = compact ? bending_force_c(c, T, k) : bending_force(c, T, k);
-        else b = bending_force(c, T, k);
-        bx[k] = b.x;
-        by[k] = b.y;
-        bz[k] = b.z;
+        V3T<P> F;
+        if constexpr (kCompact)
+          F = T.rpar ? vertex_force_rbc_r(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc)
+              : compact ? vertex_force_rbc_c(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc)
+                        : vertex_force<MODEL, TERM_ALL, P>(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc);
+        else F = vertex_force<MODEL, TERM_ALL, P>(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc, edge_f);
+        const int64_t i = base + k;
+        double f0 = (double)F.x, f1 = (double)F.y, f2 = (double)F.z;
+        if (flags & CELL_SPREAD) cap_force(i, f0, f1, f2);
+        V.f[i] = f0;
+        V.f[vs + i] = f1;
+        V.f[2 * vs + i] = f2;
       }
-    }
-    // A platelet's edges once each, for the vertices to gather: by vertex, every
-    // edge was evaluated four times and a vertex's twelve one after another
-    // (24 platelets in FP64: this kernel 51 -> 37 us).
-    P* edge_f = nullptr;
-    if constexpr (MODEL == HC_MODEL_PLT && STAGED) {
-      if (6 * (size_t)T.ne * sizeof(P) <= platelet_edge_bytes(nv, sizeof(P))) {
-        edge_f = reinterpret_cast<P*>(region);
-        for (int e = tid; e < T.ne; e += BS) platelet_edge(c, T, e, vx, vy, vz, edge_f + e, T.ne);
-      }
-    }
-    __syncthreads();
-    const P vforce = (P)vforce_sh;
-    for (int k = tid; k < nv; k += BS) {
-      V3T<P> F;
-      if constexpr (kCompact)
-        F = T.rpar ? vertex_force_rbc_r(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc)
-            : compact ? vertex_force_rbc_c(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc)
-                      : vertex_force<MODEL, TERM_ALL, P>(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc);
-      else F = vertex_force<MODEL, TERM_ALL, P>(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc, edge_f);
-      const int64_t i = base + k;
-      double f0 = (double)F.x, f1 = (double)F.y, f2 = (double)F.z;
-      if (flags & CELL_SPREAD) cap_force(i, f0, f1, f2);
-      V.f[i] = f0;
-      V.f[vs + i] = f1;
-      V.f[2 * vs + i] = f2;
     }
     __syncthreads();  // forces visible to the whole workgroup; the region is free again
   }

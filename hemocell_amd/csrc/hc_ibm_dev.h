@@ -160,6 +160,21 @@ __device__ __forceinline__ int wave_max63(int v) {
   v = max(v, dpp_move<0x142>(v));
   return max(v, dpp_move<0x143>(v));
 }
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_moved(double v) {  // 0 in lanes without a source and rows not in ROWS
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+// lane 63 gets the wavefront's sum, always added in the same order
+__device__ __forceinline__ double wave_sum63(double v) {
+  v += dpp_moved<0x111, 0xf>(v);
+  v += dpp_moved<0x112, 0xf>(v);
+  v += dpp_moved<0x114, 0xf>(v);
+  v += dpp_moved<0x118, 0xf>(v);
+  v += dpp_moved<0x142, 0xa>(v);
+  return v + dpp_moved<0x143, 0xc>(v);
+}
 // The workgroup's bounds from its threads' bounds, in LDS: reduced over each
 // wavefront first, then one LDS atomic per wavefront and bound.  With an atomic
 // per thread the lanes of a wavefront queue at one LDS word: 35000 of the 158000

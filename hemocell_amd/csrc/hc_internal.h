@@ -43,9 +43,9 @@ struct TypeHost {
   bool padded = false;          // every list fits kPadW / kPadB
   std::vector<int32_t> vtri4p, vedge4p, vbendp;  // nv*kPadW int4, nv*kPadW int4, nv*kPadB int
   // per padded slot: the rest area of its triangle, the rest length of its edge and
-  // the ring size of its bending contributor (addresses known from the vertex alone)
+  // one over the ring size of its bending contributor (addresses known from the vertex alone)
   std::vector<double> vtri_aeq, vedge_l0, vbend_n;
-  // Compact copies for the FP32 RBC kernels (padded lists, nv < 65535): per vertex
+  // Compact copies for the RBC and WBC kernels (padded lists, nv < 65535): per vertex
   // and slot j < kPadW one uint4 {corner0 | corner1 << 16, corner2 | edge partner
   // << 16, rest area (float bits), rest length (float bits)} of its j-th triangle
   // and j-th edge (0xFFFF: none); per bending slot j < kPadB the contributor i |
@@ -54,14 +54,15 @@ struct TypeHost {
   // Edges are stored from the vertex's side: the force of an edge on its second
   // end, -F(b - a), equals F(a - b) up to the rounding of fused multiply-adds.
   std::vector<uint32_t> cslot, cbend, cring;
-  // Ring-ordered tables for the FP32 RBC staged kernel, built when every vertex's
+  // Ring-ordered tables for the staged kernels, built when every vertex's
   // triangles are (v, ring[j], ring[j+1]) up to rotation (the ring is walked along
   // the triangles' winding, so this holds for a closed, consistently wound mesh),
   // its edges go to ring[j] and its bending contributors are v and its ring: per
   // vertex 12 floats (rest areas of triangles j = 0..5, then rest lengths of edges
-  // j) and one word: ring size | ring size of ring[j] << (4 + 3j).
+  // j) and one word: ring size | ring size of ring[j] << (4 + 3j).  For the FP64
+  // kernels the ids of triangles and edges j, 16 bits each: two uint4 per vertex.
   std::vector<float> rpar;
-  std::vector<uint32_t> rnb;
+  std::vector<uint32_t> rnb, rid;
   hc_model_params p{};
   int timescale = 1;
 };
@@ -84,6 +85,7 @@ struct TypeDev {
   const uint32_t* cbend;
   const float4* rpar;  // ring-ordered FP32 tables (null when not built)
   const uint32_t* rnb;
+  const uint4* rid;
   double volume_eq, area_mean_eq, edge_mean_eq;
   double k_link, k_bend, k_volume, k_area, eta_m, k_inner_rigid, k_cyto, core_radius, radius;
 };

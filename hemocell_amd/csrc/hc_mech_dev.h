@@ -102,14 +102,10 @@ __device__ __forceinline__ V3T<M> unit_normal(V3T<M> v0, V3T<M> v1, V3T<M> v2) {
   return n;
 }
 
-// bending force of vertex i from its ordered 1-ring (rbcHighOrderModel.cpp:127-166)
+// bending force of vertex i from its ordered 1-ring R[0..nr) (rbcHighOrderModel.cpp:127-166)
 template <typename M>
-__device__ V3T<M> bending_force(const CellViewT<M>& c, const TypeDev& T, int i) {
-  const int nr = T.nring[i];
-  // the ring (at most 6 entries, stored 6 wide) is loaded at once
-  int R[6];
-#pragma unroll
-  for (int j = 0; j < 6; ++j) R[j] = T.ring[6 * i + j];
+__device__ __forceinline__ V3T<M> bending_of_ring(const CellViewT<M>& c, const TypeDev& T, int i, const int (&R)[6],
+                                                  int nr) {
   const M patch_eq = (M)T.patch_dist_eq[i];
   M s0 = M(0), s1 = M(0), s2 = M(0);
 #pragma unroll
@@ -145,6 +141,14 @@ __device__ V3T<M> bending_force(const CellViewT<M>& c, const TypeDev& T, int i) 
   const M dDev = mdiv(ndev - patch_eq, (M)T.edge_mean_eq);
   const M s = (M)T.k_bend * (dDev + mdiv(dDev, mabs(M(MaxCellBendingAngle) - dDev * dDev)));
   return {pn.x * s, pn.y * s, pn.z * s};
+}
+template <typename M>
+__device__ V3T<M> bending_force(const CellViewT<M>& c, const TypeDev& T, int i) {
+  // the ring (at most 6 entries, stored 6 wide) is loaded at once
+  int R[6];
+#pragma unroll
+  for (int j = 0; j < 6; ++j) R[j] = T.ring[6 * i + j];
+  return bending_of_ring<M>(c, T, i, R, T.nring[i]);
 }
 
 // Force terms, as the reference's models add them to force_area, force_volume,
@@ -192,6 +196,173 @@ __device__ __forceinline__ void platelet_edge(const CellViewT<M>& c, const TypeD
   out[3 * stride] = ((n1.x + n2.x) * fm) * M(0.5);
   out[4 * stride] = ((n1.y + n2.y) * fm) * M(0.5);
   out[5 * stride] = ((n1.z + n2.z) * fm) * M(0.5);
+}
+
+// inner links of vertex k, inner-edge order
+template <int MODEL, typename M>
+__device__ __forceinline__ void inner_forces(const CellViewT<M>& c, const TypeDev& T, int k, M& F0, M& F1, M& F2) {
+  for (int e = T.vinner_off[k]; e < T.vinner_off[k + 1]; ++e) {
+    const int ie = T.vinner[e] >> 1, end = T.vinner[e] & 1;
+    const V3T<M> pa = c.pos(T.inner[2 * ie]), pb = c.pos(T.inner[2 * ie + 1]);
+    const V3T<M> ev = pb - pa;
+    const M len = normp(ev);
+    const V3T<M> uv = {mdiv(ev.x, len), mdiv(ev.y, len), mdiv(ev.z, len)};
+    if (MODEL == HC_MODEL_PLT) {
+      const M l0 = (M)T.inner_len_eq[ie];
+      const M ef = mdiv(len - l0, l0);
+      const M fs = (M)T.k_link * M(5.0) * ef;
+      const V3T<M> fl = {uv.x * fs, uv.y * fs, uv.z * fs};
+      if (end == 0) { F0 += fl.x; F1 += fl.y; F2 += fl.z; }
+      else { F0 -= fl.x; F1 -= fl.y; F2 -= fl.z; }
+    } else if (MODEL == HC_MODEL_WBC) {
+      const M rad = (M)T.radius, core = (M)T.core_radius;
+      if (len < 2 * rad) {
+        const M s = M(1) - mdiv(len, 2 * rad);
+        const M kc = (M)T.k_cyto;
+        const V3T<M> fl = {(uv.x * s) * kc, (uv.y * s) * kc, (uv.z * s) * kc};
+        if (end == 0) { F0 -= fl.x; F1 -= fl.y; F2 -= fl.z; }
+        else { F0 += fl.x; F1 += fl.y; F2 += fl.z; }
+      }
+      if (len < 2 * core) {
+        const M s = 1 - mdiv(len, 2 * core);
+        const M kr = (M)T.k_inner_rigid;
+        const V3T<M> fl = {(uv.x * s) * kr, (uv.y * s) * kr, (uv.z * s) * kr};
+        if (end == 0) { F0 -= fl.x; F1 -= fl.y; F2 -= fl.z; }
+        else { F0 += fl.x; F1 += fl.y; F2 += fl.z; }
+      }
+    }
+  }
+}
+
+// The FP64 mechanics of a staged RBC or WBC evaluates what needs a root or a
+// quotient once per triangle and edge, into LDS, and gathers it per vertex: the
+// vertices' own evaluation (vertex_force) takes every triangle three and every edge
+// two times over, ~2400 FP64 instructions per wavefront of vertices.
+
+// k_area (d + d / |0.09 - d^2|), d the relative change of triangle t's area
+template <typename M>
+__device__ __forceinline__ M triangle_factor(const CellViewT<M>& c, const TypeDev& T, int t) {
+  const V3T<M> v0 = c.pos(T.tri[3 * t]), v1 = c.pos(T.tri[3 * t + 1]), v2 = c.pos(T.tri[3 * t + 2]);
+  const M a_eq = (M)T.tri_area_eq[t];
+  const M area = M(0.5) * normp(crossp(v1 - v0, v2 - v0));
+  const M ar = mdiv(area - a_eq, a_eq);
+  return (M)T.k_area * (ar + mdiv(ar, mabs(M(MaxCellSurfaceAreaChange) - ar * ar)));
+}
+
+// link and membrane viscosity force of edge e over its length: its force on either
+// end is this times the separation to the other
+template <typename M>
+__device__ __forceinline__ M edge_factor(const CellViewT<M>& c, const TypeDev& T, int e, const M* vx, const M* vy,
+                                         const M* vz, bool visc) {
+  const int a = T.edge[2 * e], b = T.edge[2 * e + 1];
+  const M l0 = (M)T.edge_len_eq[e];
+  const V3T<M> ev = c.pos(b) - c.pos(a);
+  const M len = normp(ev);
+  const M il = mrcp(len);
+  const M ef = mdiv(len - l0, l0);
+  M f = (M)T.k_link * (ef + mdiv(ef, mabs(M(MaxCellPersistenceLength) - ef * ef)));
+  if (visc) {
+    const V3T<M> rv = {vx[b] - vx[a], vy[b] - vy[a], vz[b] - vz[a]};
+    const M fv = (dotp(rv, ev) * il) * (M)T.eta_m, most = M(FORCE_LIMIT / 4.0);
+    f += fv > most ? most : (fv < -most ? -most : fv);
+  }
+  return f * il;
+}
+
+// entry j of eight 16-bit entries
+__device__ __forceinline__ int ring_entry(const uint4& r, int j) {
+  const uint32_t w = j < 2 ? r.x : (j < 4 ? r.y : r.z);
+  return (int)((w >> (16 * (j & 1))) & 0xFFFFu);
+}
+
+// One vertex's 1-ring (TypeHost::cring, rnb): its size 3..6 and the neighbours
+struct RingOf {
+  int nr, R[6];
+  uint32_t sizes;
+  __device__ __forceinline__ RingOf(const TypeDev& T, int k) {
+    const uint4 rq = T.cring[k];
+    sizes = T.rnb[k];
+    nr = (int)(sizes & 7u);
+#pragma unroll
+    for (int j = 0; j < 6; ++j) R[j] = j < nr ? ring_entry(rq, j) : k;
+  }
+  // one over the ring size of neighbour j
+  template <typename M>
+  __device__ __forceinline__ M inverse_size(int j) const {
+    const uint32_t n = (sizes >> (4 + 3 * j)) & 7u;
+    return n == 6 ? M(1) / M(6) : (n == 5 ? M(1) / M(5) : (n == 4 ? M(1) / M(4) : mrcp((M)n)));
+  }
+};
+
+// area and volume forces of vertex k: (centroid - x_k) times the triangle's factor,
+// and vforce times area and unit normal (half the cross product) over the mean area
+template <typename M>
+__device__ __forceinline__ void gather_triangles(const CellViewT<M>& c, const TypeDev& T, const RingOf& g, int k,
+                                                 const M* factor, M vforce, M& F0, M& F1, M& F2) {
+  const uint4 id = T.rid[2 * k];
+  const V3T<M> xk = c.pos(k);
+  V3T<M> d[6];
+  M f[6];
+#pragma unroll
+  for (int j = 0; j < 6; ++j) {
+    d[j] = c.pos(g.R[j]) - xk;
+    f[j] = factor[ring_entry(id, j)];
+  }
+  M A0 = M(0), A1 = M(0), A2 = M(0), B0 = M(0), B1 = M(0), B2 = M(0);
+#pragma unroll
+  for (int j = 0; j < 6; ++j) {
+    if (j >= 3 && j >= g.nr) break;
+    const V3T<M> a = d[j];
+    V3T<M> b = d[j < 5 ? j + 1 : 0];
+    if (j + 1 >= g.nr) b = d[0];
+    const V3T<M> n = crossp(a, b);
+    A0 += (a.x + b.x) * f[j];
+    A1 += (a.y + b.y) * f[j];
+    A2 += (a.z + b.z) * f[j];
+    B0 += n.x;
+    B1 += n.y;
+    B2 += n.z;
+  }
+  const M s = mdiv(M(0.5) * vforce, (M)T.area_mean_eq);
+  constexpr M third = M(1.0 / 3.0);
+  F0 = A0 * third + B0 * s;
+  F1 = A1 * third + B1 * s;
+  F2 = A2 * third + B2 * s;
+}
+
+// bending forces on vertex k: its own and -F_i / n_i of its neighbours
+template <typename M>
+__device__ __forceinline__ void gather_bending(const RingOf& g, int k, const M* bx, const M* by, const M* bz, M& F0,
+                                               M& F1, M& F2) {
+  F0 += bx[k];
+  F1 += by[k];
+  F2 += bz[k];
+#pragma unroll
+  for (int j = 0; j < 6; ++j) {
+    if (j >= 3 && j >= g.nr) break;
+    const M in = g.template inverse_size<M>(j);
+    const int i = g.R[j];
+    F0 -= bx[i] * in;
+    F1 -= by[i] * in;
+    F2 -= bz[i] * in;
+  }
+}
+
+// link and membrane viscosity forces on vertex k
+template <typename M>
+__device__ __forceinline__ void gather_edges(const CellViewT<M>& c, const TypeDev& T, const RingOf& g, int k,
+                                             const M* factor, M& F0, M& F1, M& F2) {
+  const uint4 id = T.rid[2 * k + 1];
+  const V3T<M> xk = c.pos(k);
+#pragma unroll
+  for (int j = 0; j < 6; ++j) {
+    if (j >= 3 && j >= g.nr) break;
+    const V3T<M> d = c.pos(g.R[j]) - xk;
+    const M f = factor[ring_entry(id, j)];
+    F0 += d.x * f;
+    F1 += d.y * f;
+    F2 += d.z * f;
+  }
 }
 
 // Force on vertex k of one cell: every term gathered in the reference's order
@@ -268,14 +439,13 @@ __device__ __forceinline__ V3T<M> vertex_force(const CellViewT<M>& c, const Type
   }
   // bending: own force and -F_i/n_i of every vertex i whose 1-ring holds k, ascending i
   if (MODEL != HC_MODEL_PLT && (TERMS & TERM_BENDING)) {
-    auto bend_term = [&](const int i, const M dn) {
+    auto bend_term = [&](const int i, const M in) {
       const M b0 = bx[i], b1 = by[i], b2 = bz[i];
       if (i == k) {
         F0 += b0;
         F1 += b1;
         F2 += b2;
       } else {
-        const M in = mrcp(dn);
         F0 += -b0 * in;
         F1 += -b1 * in;
         F2 += -b2 * in;
@@ -283,18 +453,18 @@ __device__ __forceinline__ V3T<M> vertex_force(const CellViewT<M>& c, const Type
     };
     if (T.vbendp) {
       int b[kPadB];
-      M dn[kPadB];
+      M in[kPadB];
 #pragma unroll
       for (int j = 0; j < kPadB; ++j) {
         b[j] = T.vbendp[kPadB * k + j];
-        dn[j] = (M)T.vbend_n[kPadB * k + j];
+        in[j] = (M)T.vbend_n[kPadB * k + j];
       }
 #pragma unroll
       for (int j = 0; j < kPadB; ++j)
-        if (b[j] >= 0) bend_term(b[j], dn[j]);
+        if (b[j] >= 0) bend_term(b[j], in[j]);
     } else {
       for (int e = T.vbend_off[k]; e < T.vbend_off[k + 1]; ++e)
-        bend_term(T.vbend[e], (M)(unsigned)T.nring[T.vbend[e]]);
+        bend_term(T.vbend[e], mrcp((M)(unsigned)T.nring[T.vbend[e]]));
     }
   }
   // edges: link, membrane viscosity, (PLT) dihedral bending; edge order
@@ -377,38 +547,7 @@ __device__ __forceinline__ V3T<M> vertex_force(const CellViewT<M>& c, const Type
     for (int e = T.vedge_off[k]; e < T.vedge_off[k + 1]; ++e)
       edge_term(T.vedge4[e], (M)T.edge_len_eq[T.vedge4[e].x >> 2]);
   }
-  // inner links, inner-edge order
-  for (int e = T.vinner_off[k]; (TERMS & TERM_INNER) && e < T.vinner_off[k + 1]; ++e) {
-    const int ie = T.vinner[e] >> 1, end = T.vinner[e] & 1;
-    const V3T<M> pa = c.pos(T.inner[2 * ie]), pb = c.pos(T.inner[2 * ie + 1]);
-    const V3T<M> ev = pb - pa;
-    const M len = normp(ev);
-    const V3T<M> uv = {mdiv(ev.x, len), mdiv(ev.y, len), mdiv(ev.z, len)};
-    if (MODEL == HC_MODEL_PLT) {
-      const M l0 = (M)T.inner_len_eq[ie];
-      const M ef = mdiv(len - l0, l0);
-      const M fs = (M)T.k_link * M(5.0) * ef;
-      const V3T<M> fl = {uv.x * fs, uv.y * fs, uv.z * fs};
-      if (end == 0) { F0 += fl.x; F1 += fl.y; F2 += fl.z; }
-      else { F0 -= fl.x; F1 -= fl.y; F2 -= fl.z; }
-    } else if (MODEL == HC_MODEL_WBC) {
-      const M rad = (M)T.radius, core = (M)T.core_radius;
-      if (len < 2 * rad) {
-        const M s = M(1) - mdiv(len, 2 * rad);
-        const M kc = (M)T.k_cyto;
-        const V3T<M> fl = {(uv.x * s) * kc, (uv.y * s) * kc, (uv.z * s) * kc};
-        if (end == 0) { F0 -= fl.x; F1 -= fl.y; F2 -= fl.z; }
-        else { F0 += fl.x; F1 += fl.y; F2 += fl.z; }
-      }
-      if (len < 2 * core) {
-        const M s = 1 - mdiv(len, 2 * core);
-        const M kr = (M)T.k_inner_rigid;
-        const V3T<M> fl = {(uv.x * s) * kr, (uv.y * s) * kr, (uv.z * s) * kr};
-        if (end == 0) { F0 -= fl.x; F1 -= fl.y; F2 -= fl.z; }
-        else { F0 += fl.x; F1 += fl.y; F2 += fl.z; }
-      }
-    }
-  }
+  if (TERMS & TERM_INNER) inner_forces<MODEL, M>(c, T, k, F0, F1, F2);
   return {F0, F1, F2};
 }
 
@@ -418,11 +557,6 @@ __device__ __forceinline__ V3T<M> vertex_force(const CellViewT<M>& c, const Type
 // edge is taken from the vertex's side (its force on the second end, -F(b - a),
 // is F(a - b) in exact arithmetic; the multiply-adds the compiler fuses differ),
 // so one uint4 per slot carries a triangle and an edge.
-__device__ __forceinline__ int ring_entry(const uint4& r, int j) {
-  const uint32_t w = j < 2 ? r.x : (j < 4 ? r.y : r.z);
-  return (int)((w >> (16 * (j & 1))) & 0xFFFFu);
-}
-
 __device__ V3T<float> bending_force_c(const CellViewT<float>& c, const TypeDev& T, int i) {
   using M = float;
   const uint4 rq = T.cring[i];

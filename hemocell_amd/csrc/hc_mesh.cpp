@@ -436,14 +436,14 @@ bool build_type_tables(TypeHost& T, std::string& err) {
       }
       for (int e = T.vbend_off[v], j = 0; e < T.vbend_off[v + 1]; ++e, ++j) {
         T.vbendp[(size_t)v * kPadB + j] = T.vbend[e];
-        T.vbend_n[(size_t)v * kPadB + j] = (double)(unsigned)T.nring[T.vbend[e]];
+        T.vbend_n[(size_t)v * kPadB + j] = 1.0 / (double)(unsigned)T.nring[T.vbend[e]];
       }
     }
   }
   T.cslot.clear();
   T.cbend.clear();
   T.cring.clear();
-  if (T.padded && T.model == HC_MODEL_RBC && nv < 0xFFFF) {
+  if (T.padded && T.model != HC_MODEL_PLT && nv < 0xFFFF) {
     auto fbits = [](double x) {
       const float f = (float)x;
       uint32_t u;
@@ -489,9 +489,10 @@ bool build_type_tables(TypeHost& T, std::string& err) {
   }
   T.rpar.clear();
   T.rnb.clear();
+  T.rid.clear();
   if (!T.cring.empty()) {
     std::vector<float> par((size_t)nv * 12, 1.0f);
-    std::vector<uint32_t> nb((size_t)nv, 0);
+    std::vector<uint32_t> nb((size_t)nv, 0), id((size_t)nv * 8, 0);
     bool ok = true;
     for (int v = 0; v < nv && ok; ++v) {
       const int nr = T.nring[v];
@@ -519,6 +520,7 @@ bool build_type_tables(TypeHost& T, std::string& err) {
         }
         seen_t |= 1u << j;
         par[12 * (size_t)v + j] = (float)T.tri_area_eq[q[0]];
+        id[8 * (size_t)v + (j >> 1)] |= (uint32_t)q[0] << (16 * (j & 1));
       }
       for (int e = T.vedge_off[v]; ok && e < T.vedge_off[v + 1]; ++e) {
         const int code = T.vedge[e], ed = code >> 2, kind = code & 3;
@@ -530,6 +532,7 @@ bool build_type_tables(TypeHost& T, std::string& err) {
         }
         seen_e |= 1u << j;
         par[12 * (size_t)v + 6 + j] = (float)T.edge_len_eq[ed];
+        id[8 * (size_t)v + 4 + (j >> 1)] |= (uint32_t)ed << (16 * (j & 1));
       }
       const unsigned all = (1u << nr) - 1u;
       ok = ok && seen_t == all && seen_e == all && T.vbend_off[v + 1] - T.vbend_off[v] == nr + 1;
@@ -558,6 +561,7 @@ bool build_type_tables(TypeHost& T, std::string& err) {
     if (ok) {
       T.rpar.swap(par);
       T.rnb.swap(nb);
+      if (T.edge.size() / 2 < 0xFFFF && T.tri.size() / 3 < 0xFFFF) T.rid.swap(id);
     }
   }
   return true;
