@@ -1811,12 +1811,16 @@ hc_status hc_add_cell_type(hc_ctx* ctx, int model, int nv, int nt, const int32_t
     D.rpar = nullptr;
     D.rnb = nullptr;
     D.rid = nullptr;
+    // the tables of one precision's kernels only, once it is known
+    const bool f32 = !ctx->lattice_ready || fp32(ctx), f64 = !ctx->lattice_ready || !fp32(ctx);
     if (!T.rpar.empty() && !padded_off(ctx) && !ring_tables_off()) {
-      const float* pf = nullptr;
-      if ((s = upload(ctx, *tb, T.rpar, &pf)) != HC_OK) return s;
-      D.rpar = (const float4*)pf;
+      if (f32) {
+        const float* pf = nullptr;
+        if ((s = upload(ctx, *tb, T.rpar, &pf)) != HC_OK) return s;
+        D.rpar = (const float4*)pf;
+      }
       if ((s = upload(ctx, *tb, T.rnb, &D.rnb)) != HC_OK) return s;
-      if (!T.rid.empty()) {
+      if (f64 && !T.rid.empty()) {
         const uint32_t* pi = nullptr;
         if ((s = upload(ctx, *tb, T.rid, &pi)) != HC_OK) return s;
         D.rid = (const uint4*)pi;
@@ -1824,11 +1828,13 @@ hc_status hc_add_cell_type(hc_ctx* ctx, int model, int nv, int nt, const int32_t
     }
     if (!T.cslot.empty() && !padded_off(ctx)) {
       const uint32_t* pc = nullptr;
-      if ((s = upload(ctx, *tb, T.cslot, &pc)) != HC_OK) return s;
-      D.cslot = (const uint4*)pc;
       if ((s = upload(ctx, *tb, T.cring, &pc)) != HC_OK) return s;
       D.cring = (const uint4*)pc;
-      if ((s = upload(ctx, *tb, T.cbend, &D.cbend)) != HC_OK) return s;
+      if (f32 && !D.rpar) {
+        if ((s = upload(ctx, *tb, T.cslot, &pc)) != HC_OK) return s;
+        D.cslot = (const uint4*)pc;
+        if ((s = upload(ctx, *tb, T.cbend, &D.cbend)) != HC_OK) return s;
+      }
     }
     if (T.padded && !padded_off(ctx)) {
       if ((s = upload(ctx, *tb, T.vtri4p, &p4)) != HC_OK) return s;

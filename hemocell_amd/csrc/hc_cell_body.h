@@ -425,10 +425,11 @@ __device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev
     if (!once) {
       __syncthreads();
       if (tid == 0) vforce_sh = volume_force();
-      // FP32 RBC: the ring-ordered tables, else the compact per-slot ones (both
-      // built beside the padded tables)
-      constexpr bool kCompact = MODEL == HC_MODEL_RBC && std::is_same<P, float>::value;
-      const bool compact = kCompact && T.cslot != nullptr;
+      // FP32 RBC and WBC: the ring-ordered tables, else the compact per-slot ones
+      // (both built beside the padded tables, whose entries lie 112 bytes apart: a
+      // 642-vertex WBC's forces took 22 of 77 kcycles with them, 13 with the rings)
+      constexpr bool kCompact = MODEL != HC_MODEL_PLT && std::is_same<P, float>::value;
+      const bool compact = kCompact && T.cring != nullptr;
       if (MODEL != HC_MODEL_PLT) {
         for (int k = tid; k < nv; k += BS) {
           V3T<P> b;
@@ -453,11 +454,12 @@ __device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev
       const P vforce = (P)vforce_sh;
       for (int k = tid; k < nv; k += BS) {
         V3T<P> F;
-        if constexpr (kCompact)
-          F = T.rpar ? vertex_force_rbc_r(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc)
-              : compact ? vertex_force_rbc_c(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc)
-                        : vertex_force<MODEL, TERM_ALL, P>(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc);
-        else F = vertex_force<MODEL, TERM_ALL, P>(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc, edge_f);
+        if constexpr (kCompact) {
+          if (T.rpar) F = vertex_force_ring(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc);
+          else if (compact) F = vertex_force_compact(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc);
+          else F = vertex_force<MODEL, TERM_ALL & ~TERM_INNER, P>(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc);
+          inner_forces<MODEL, P>(c, T, k, F.x, F.y, F.z);
+        } else F = vertex_force<MODEL, TERM_ALL, P>(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc, edge_f);
         const int64_t i = base + k;
         double f0 = (double)F.x, f1 = (double)F.y, f2 = (double)F.z;
         if (flags & CELL_SPREAD) cap_force(i, f0, f1, f2);

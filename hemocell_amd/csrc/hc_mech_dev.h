@@ -551,9 +551,9 @@ __device__ __forceinline__ V3T<M> vertex_force(const CellViewT<M>& c, const Type
   return {F0, F1, F2};
 }
 
-// The FP32 RBC kernels' bending and vertex forces over the compact tables
+// The FP32 RBC and WBC kernels' bending and vertex forces (but for inner links) over the compact tables
 // (TypeHost::cslot / cbend / cring): the terms, their order and their operations
-// are those of bending_force and vertex_force<HC_MODEL_RBC, TERM_ALL, float>; an
+// are those of bending_force and vertex_force<HC_MODEL_RBC>; an
 // edge is taken from the vertex's side (its force on the second end, -F(b - a),
 // is F(a - b) in exact arithmetic; the multiply-adds the compiler fuses differ),
 // so one uint4 per slot carries a triangle and an edge.
@@ -604,7 +604,7 @@ __device__ V3T<float> bending_force_c(const CellViewT<float>& c, const TypeDev& 
   return {pn.x * s, pn.y * s, pn.z * s};
 }
 
-__device__ __forceinline__ V3T<float> vertex_force_rbc_c(const CellViewT<float>& c, const TypeDev& T, int k,
+__device__ __forceinline__ V3T<float> vertex_force_compact(const CellViewT<float>& c, const TypeDev& T, int k,
                                                           float vforce, const float* bx, const float* by,
                                                           const float* bz, const float* vx, const float* vy,
                                                           const float* vz, bool visc) {
@@ -705,7 +705,7 @@ __device__ __forceinline__ V3T<float> vertex_force_rbc_c(const CellViewT<float>&
   return {F0, F1, F2};
 }
 
-// The FP32 RBC kernels' vertex force over the ring-ordered tables (TypeHost::rpar
+// The FP32 RBC and WBC kernels' vertex force (but for inner links) over the ring-ordered tables (TypeHost::rpar
 // / rnb): the terms of vertex_force<HC_MODEL_RBC>, summed around the 1-ring.
 // Triangle j is (k, ring[j], ring[j+1]) and edge j is (k, ring[j]), so each
 // neighbour's position is read once and enters as its offset d_j from vertex k:
@@ -713,7 +713,7 @@ __device__ __forceinline__ V3T<float> vertex_force_rbc_c(const CellViewT<float>&
 // its area is half the cross product.  The sums run in ring order (own bending
 // force first) rather than in the reference's triangle, contributor and edge
 // order: the same force up to FP32 rounding.
-__device__ __forceinline__ V3T<float> vertex_force_rbc_r(const CellViewT<float>& c, const TypeDev& T, int k,
+__device__ __forceinline__ V3T<float> vertex_force_ring(const CellViewT<float>& c, const TypeDev& T, int k,
                                                           float vforce, const float* bx, const float* by,
                                                           const float* bz, const float* vx, const float* vy,
                                                           const float* vz, bool visc) {
