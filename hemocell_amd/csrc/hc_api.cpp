@@ -817,16 +817,19 @@ hc_status do_cell_step(hc_ctx* ctx, int do_interp, bool spread) {
     if ((ctx->iter % tb.host.timescale) == 0) flags |= CELL_FLAG_MECH;
     const bool few = tb.ncells < ctx->n_cu;
     int block = cell_threads(ctx, tb.host.model, few);
-    // while compute units are left over beside the main type, a large side cell
-    // takes one for itself with its positions in LDS: one 2562-vertex WBC beside
-    // 242 RBC, 350 -> 121 us per step
-    const bool gpos = k != 0 && nside > 0 && ctx->side_gpos && 3 * (size_t)tb.host.nv * sizeof(double) > 32768 &&
-                      act[0]->ncells + tb.ncells > ctx->n_cu;
+    // A large side cell's positions are doubles in either precision, in global memory
+    // or in LDS, so that its mechanics do not change with the number of cells.  While
+    // compute units are left over beside the main type it takes one for itself with
+    // the positions in LDS (one 2562-vertex WBC beside 216 RBC: 442 -> 269 us per step
+    // in FP64, 329 -> 174 in FP32; 130 with float offsets, whose forces are 4e-4 off).
+    const bool large = k != 0 && nside > 0 && 3 * (size_t)tb.host.nv * sizeof(double) > 32768;
+    const bool gpos = large && ctx->side_gpos && act[0]->ncells + tb.ncells > ctx->n_cu;
+    const CellPositions pos = gpos ? POS_GLOBAL : (large ? POS_LDS_DOUBLE : POS_LDS);
     const int box = spread_box_bytes(ctx, tb.host.model, few && !gpos);
     if (gpos) block = 256;
     HC_TRY(launch_cell_step<R>(st, vdev(ctx), tb.dev, tb.d_cells, tb.ncells, ctx->d_cell_base, (const R*)ctx->ufield,
                                ctx->type, ctx->L, (R*)ctx->Fibm[1 - ctx->cur], ctx->d_extra_dense, ctx->bend,
-                               ctx->f_limit, flags, box, ctx->lds_device, ctx->d_wall_hits, block, gpos),
+                               ctx->f_limit, flags, box, ctx->lds_device, ctx->d_wall_hits, block, pos),
            "cell_step");
   }
   for (int j = 0; j < nside; ++j) {

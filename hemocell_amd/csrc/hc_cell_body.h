@@ -760,7 +760,7 @@ template <typename R, int M, int B>
 static hipError_t launch_cell(hipStream_t s, const VertexDev& V, const TypeDev& T, const int32_t* cells, int ncells,
                               const int64_t* cell_base, const R* uf, const uint8_t* type, const LatticeDev& L, R* Fnext,
                               const double* extra, double* scratch, double f_limit, int flags, int box_bytes,
-                              int lds_device, unsigned long long* wall_hits, bool gpos,
+                              int lds_device, unsigned long long* wall_hits, CellPositions pos,
                               const CellCase* multi = nullptr) {
   static const size_t st_staged = std::max(static_lds(k_cell_step<R, M, B, true, false>),
                                            static_lds(k_cell_step_multi<R, M, B, true, false>));
@@ -769,9 +769,10 @@ static hipError_t launch_cell(hipStream_t s, const VertexDev& V, const TypeDev& 
   static const size_t st_gpos = static_lds(k_cell_step<R, M, B, false, true>);
   const bool visc = (T.model != HC_MODEL_RBC) || (T.eta_m != 0.0);
   // the staged kernel's position scalar: float offsets in the FP32-shifted form
-  const CellLdsPlan plan = cell_lds_plan(T.model, T.nv, visc, sizeof(MechT<R, true, false>), (size_t)box_bytes,
-                                         (size_t)lds_device, st_staged, st_plain, st_gpos, gpos);
+  const CellLdsPlan plan = cell_lds_layout(T.model, T.nv, visc, sizeof(MechT<R, true, false>), (size_t)box_bytes,
+                                           (size_t)lds_device, st_staged, st_plain, st_gpos, pos);
   if (!plan.ok) return hipErrorInvalidConfiguration;
+  const bool gpos = pos == POS_GLOBAL;
   const bool staged = plan.staged;
   const int box_nodes = plan.box_nodes;
   const size_t dyn = plan.dyn;
@@ -801,7 +802,7 @@ template <typename R>
 hipError_t launch_cell_step(hipStream_t s, const VertexDev& V, const TypeDev& T, const int32_t* cells, int ncells,
                             const int64_t* cell_base, const R* uf, const uint8_t* type, const LatticeDev& L,
                             R* Fnext, const double* extra, double* scratch, double f_limit, int flags, int box_bytes,
-                            int lds_device, unsigned long long* wall_hits, int block, bool gpos) {
+                            int lds_device, unsigned long long* wall_hits, int block, CellPositions pos) {
   if (ncells <= 0) return hipSuccess;
   // threads per cell for the RBC and WBC meshes: 256, 512 or 1024; a block whose
   // static LDS leaves too little room for the cell falls back to a smaller one
@@ -809,7 +810,7 @@ hipError_t launch_cell_step(hipStream_t s, const VertexDev& V, const TypeDev& T,
 #define HC_CELL(M, B)                                                                                                \
   if (e == hipErrorInvalidConfiguration)                                                                             \
     e = launch_cell<R, M, B>(s, V, T, cells, ncells, cell_base, uf, type, L, Fnext, extra, scratch, f_limit, flags, \
-                             box_bytes, lds_device, wall_hits, gpos);
+                             box_bytes, lds_device, wall_hits, pos);
   switch (T.model) {
     case HC_MODEL_RBC:
       if (block >= 1024) HC_CELL(HC_MODEL_RBC, 1024)
@@ -831,9 +832,9 @@ hipError_t launch_cell_step(hipStream_t s, const VertexDev& V, const TypeDev& T,
 #undef HC_CELL
   // a mesh whose positions do not fit the workgroup's LDS at any block (a
   // 2562-vertex WBC on a 64 KB device) keeps them in global memory
-  if (e == hipErrorInvalidConfiguration && !gpos)
+  if (e == hipErrorInvalidConfiguration && pos != POS_GLOBAL)
     return launch_cell_step<R>(s, V, T, cells, ncells, cell_base, uf, type, L, Fnext, extra, scratch, f_limit, flags,
-                               box_bytes, lds_device, wall_hits, 256, true);
+                               box_bytes, lds_device, wall_hits, 256, POS_GLOBAL);
   return e;
 }
 
@@ -900,7 +901,7 @@ hipError_t launch_cell_step_multi(hipStream_t s, const TypeDev& T, const CellCas
 #define HC_CELL(M, B)                                                                                             \
   if (e == hipErrorInvalidConfiguration)                                                                          \
     e = launch_cell<R, M, B>(s, V, T, nullptr, ncells, nullptr, nullptr, nullptr, L, nullptr, nullptr, nullptr, 0.0, \
-                             0, box_bytes, lds_device, nullptr, false, cases);
+                             0, box_bytes, lds_device, nullptr, POS_LDS, cases);
   switch (T.model) {
     case HC_MODEL_RBC:
       if (block >= 1024) HC_CELL(HC_MODEL_RBC, 1024)

@@ -9,7 +9,7 @@ template hipError_t launch_cell_step_multi<double>(hipStream_t, const TypeDev&, 
 template hipError_t launch_cell_step<double>(hipStream_t, const VertexDev&, const TypeDev&, const int32_t*, int,
                                              const int64_t*, const double*, const uint8_t*, const LatticeDev&, double*,
                                              const double*, double*, double, int, int, int, unsigned long long*, int,
-                                             bool);
+                                             CellPositions);
 template hipError_t launch_cell_step_mixed<double>(hipStream_t, const VertexDev&, const TypeDev*, const TypeDev*, int,
                                               const int*, const int2*, int, unsigned int*, int, const int64_t*,
                                               const double*, const uint8_t*, const LatticeDev&, double*, const double*,

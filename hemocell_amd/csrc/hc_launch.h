@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include "hc_internal.h"
+#include "hc_lds_plan.h"
 
 namespace hcg {
 
@@ -87,7 +88,7 @@ template <typename R>
 hipError_t launch_cell_step(hipStream_t s, const VertexDev& V, const TypeDev& T, const int32_t* cells, int ncells,
                             const int64_t* cell_base, const R* uf, const uint8_t* type, const LatticeDev& L,
                             R* Fnext, const double* extra, double* scratch, double f_limit, int flags, int box_bytes,
-                            int lds_device, unsigned long long* wall_hits, int block, bool gpos = false);
+                            int lds_device, unsigned long long* wall_hits, int block, CellPositions pos = POS_LDS);
 
 // all cell types in one persistent launch (hc_cell_*.hip): a queue of (cell,
 // type index) entries, the types with most vertices first; flags per type

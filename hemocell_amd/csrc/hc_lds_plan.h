@@ -70,6 +70,19 @@ inline CellLdsPlan cell_lds_plan(int model, int nv, bool visc, size_t psize, siz
   return p;
 }
 
+// Where a launch keeps the positions: in LDS (the FP32-shifted form's staged kernels
+// as float offsets, the others as doubles), in LDS as doubles, or in global memory.
+enum CellPositions { POS_LDS = 0, POS_LDS_DOUBLE = 1, POS_GLOBAL = 2 };
+
+// cell_lds_plan for a launch that may ask for positions as doubles, which with float
+// offsets in the staged layout (psize 4) leaves the plain one.
+inline CellLdsPlan cell_lds_layout(int model, int nv, bool visc, size_t psize, size_t box_bytes, size_t lds_device,
+                                   size_t st_staged, size_t st_plain, size_t st_gpos, CellPositions pos) {
+  const bool plain = pos == POS_LDS_DOUBLE && psize != sizeof(double);
+  return cell_lds_plan(model, nv, visc, psize, box_bytes, lds_device, plain ? lds_device : st_staged, st_plain,
+                       st_gpos, pos == POS_GLOBAL);
+}
+
 // The persistent mixed launch: one dynamic size for every type (staged RBC and
 // platelets, WBCs with positions in global memory), each type's box filling
 // what its own fixed part and list leave.  Returns the dynamic bytes, 0 when
