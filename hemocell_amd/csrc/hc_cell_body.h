@@ -327,7 +327,8 @@ __device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev
     // evaluated at once, then gathered; otherwise one after the other, with the
     // vertices' sums in V.f between.  The sums are the same either way.  One
     // RBC 57 -> 52 us per step; 120 x 136 x 250 nodes with 1886 RBC 765 -> 743.
-    constexpr bool kOnce = MODEL != HC_MODEL_PLT && STAGED && std::is_same<P, double>::value;
+    constexpr bool kFactors = MODEL != HC_MODEL_PLT && std::is_same<R, double>::value;
+    constexpr bool kOnce = kFactors && STAGED;
     const bool once = kOnce && T.rid;  // at most 2 nv triangles and 3 nv edges
     const bool apart = 3 * nv + T.nt + T.ne <= 3 * box_nodes;
     P* const tri_f = reinterpret_cast<P*>(region) + (apart ? 3 * nv : 0);
@@ -454,7 +455,10 @@ __device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev
       const P vforce = (P)vforce_sh;
       for (int k = tid; k < nv; k += BS) {
         V3T<P> F;
-        if constexpr (kCompact) {
+        if constexpr (kFactors && !STAGED) {
+          if (T.rid) F = vertex_force_factors<MODEL, P>(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc);
+          else F = vertex_force<MODEL, TERM_ALL, P>(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc);
+        } else if constexpr (kCompact) {
           if (T.rpar) F = vertex_force_ring(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc);
           else if (compact) F = vertex_force_compact(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc);
           else F = vertex_force<MODEL, TERM_ALL & ~TERM_INNER, P>(c, T, k, vforce, bx, by, bz, vx, vy, vz, visc);
@@ -766,7 +770,10 @@ static hipError_t launch_cell(hipStream_t s, const VertexDev& V, const TypeDev& 
                                            static_lds(k_cell_step_multi<R, M, B, true, false>));
   static const size_t st_plain = std::max(static_lds(k_cell_step<R, M, B, false, false>),
                                           static_lds(k_cell_step_multi<R, M, B, false, false>));
-  static const size_t st_gpos = static_lds(k_cell_step<R, M, B, false, true>);
+  // positions in global memory: 256 threads at most
+  constexpr bool kGlobal = B <= 256;
+  static const size_t st_gpos = kGlobal ? static_lds(k_cell_step<R, M, kGlobal ? B : 256, false, true>) : 0;
+  if (pos == POS_GLOBAL && !kGlobal) return hipErrorInvalidConfiguration;
   const bool visc = (T.model != HC_MODEL_RBC) || (T.eta_m != 0.0);
   // the staged kernel's position scalar: float offsets in the FP32-shifted form
   const CellLdsPlan plan = cell_lds_layout(T.model, T.nv, visc, sizeof(MechT<R, true, false>), (size_t)box_bytes,
@@ -790,8 +797,8 @@ static hipError_t launch_cell(hipStream_t s, const VertexDev& V, const TypeDev& 
     hipLaunchKernelGGL((k_cell_step<R, M, B, true, false>), dim3((unsigned)ncells), dim3(B), dyn, s, V, T, cells,
                        cell_base, uf, type, L, Fnext, extra, scratch, f_limit, flags, box_nodes, wall_hits);
   else if (gpos)
-    hipLaunchKernelGGL((k_cell_step<R, M, B, false, true>), dim3((unsigned)ncells), dim3(B), dyn, s, V, T, cells,
-                       cell_base, uf, type, L, Fnext, extra, scratch, f_limit, flags, box_nodes, wall_hits);
+    hipLaunchKernelGGL((k_cell_step<R, M, kGlobal ? B : 256, false, true>), dim3((unsigned)ncells), dim3(B), dyn, s, V,
+                       T, cells, cell_base, uf, type, L, Fnext, extra, scratch, f_limit, flags, box_nodes, wall_hits);
   else
     hipLaunchKernelGGL((k_cell_step<R, M, B, false, false>), dim3((unsigned)ncells), dim3(B), dyn, s, V, T, cells,
                        cell_base, uf, type, L, Fnext, extra, scratch, f_limit, flags, box_nodes, wall_hits);

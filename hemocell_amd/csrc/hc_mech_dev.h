@@ -237,7 +237,10 @@ __device__ __forceinline__ void inner_forces(const CellViewT<M>& c, const TypeDe
 // The FP64 mechanics of a staged RBC or WBC evaluates what needs a root or a
 // quotient once per triangle and edge, into LDS, and gathers it per vertex: the
 // vertices' own evaluation (vertex_force) takes every triangle three and every edge
-// two times over, ~2400 FP64 instructions per wavefront of vertices.
+// two times over, ~2400 FP64 instructions per wavefront of vertices.  The layouts
+// without room for the factors evaluate them where they are gathered
+// (vertex_force_factors): the same operations in the same order, so that a cell's
+// forces do not depend, to the bit, on the layout its launch takes.
 
 // k_area (d + d / |0.09 - d^2|), d the relative change of triangle t's area
 template <typename M>
@@ -297,6 +300,27 @@ struct RingOf {
 // area and volume forces of vertex k: (centroid - x_k) times the triangle's factor,
 // and vforce times area and unit normal (half the cross product) over the mean area
 template <typename M>
+struct TriangleSum {
+  M A0 = M(0), A1 = M(0), A2 = M(0), B0 = M(0), B1 = M(0), B2 = M(0);
+  // the triangle with the offsets a and b of its other corners from the vertex
+  __device__ __forceinline__ void add(const V3T<M>& a, const V3T<M>& b, M factor) {
+    const V3T<M> n = crossp(a, b);
+    A0 += (a.x + b.x) * factor;
+    A1 += (a.y + b.y) * factor;
+    A2 += (a.z + b.z) * factor;
+    B0 += n.x;
+    B1 += n.y;
+    B2 += n.z;
+  }
+  __device__ __forceinline__ void force(const TypeDev& T, M vforce, M& F0, M& F1, M& F2) const {
+    const M s = mdiv(M(0.5) * vforce, (M)T.area_mean_eq);
+    constexpr M third = M(1.0 / 3.0);
+    F0 = A0 * third + B0 * s;
+    F1 = A1 * third + B1 * s;
+    F2 = A2 * third + B2 * s;
+  }
+};
+template <typename M>
 __device__ __forceinline__ void gather_triangles(const CellViewT<M>& c, const TypeDev& T, const RingOf& g, int k,
                                                  const M* factor, M vforce, M& F0, M& F1, M& F2) {
   const uint4 id = T.rid[2 * k];
@@ -308,26 +332,15 @@ __device__ __forceinline__ void gather_triangles(const CellViewT<M>& c, const Ty
     d[j] = c.pos(g.R[j]) - xk;
     f[j] = factor[ring_entry(id, j)];
   }
-  M A0 = M(0), A1 = M(0), A2 = M(0), B0 = M(0), B1 = M(0), B2 = M(0);
+  TriangleSum<M> sum;
 #pragma unroll
   for (int j = 0; j < 6; ++j) {
     if (j >= 3 && j >= g.nr) break;
-    const V3T<M> a = d[j];
     V3T<M> b = d[j < 5 ? j + 1 : 0];
     if (j + 1 >= g.nr) b = d[0];
-    const V3T<M> n = crossp(a, b);
-    A0 += (a.x + b.x) * f[j];
-    A1 += (a.y + b.y) * f[j];
-    A2 += (a.z + b.z) * f[j];
-    B0 += n.x;
-    B1 += n.y;
-    B2 += n.z;
+    sum.add(d[j], b, f[j]);
   }
-  const M s = mdiv(M(0.5) * vforce, (M)T.area_mean_eq);
-  constexpr M third = M(1.0 / 3.0);
-  F0 = A0 * third + B0 * s;
-  F1 = A1 * third + B1 * s;
-  F2 = A2 * third + B2 * s;
+  sum.force(T, vforce, F0, F1, F2);
 }
 
 // bending forces on vertex k: its own and -F_i / n_i of its neighbours
@@ -363,6 +376,38 @@ __device__ __forceinline__ void gather_edges(const CellViewT<M>& c, const TypeDe
     F1 += d.y * f;
     F2 += d.z * f;
   }
+}
+
+// The force on vertex k from factors evaluated here, summed as the staged kernels
+// gather theirs.  One triangle or edge after another: all at once take the registers
+// of a wavefront per SIMD (166 VGPRs, positions in global memory).
+template <int MODEL, typename M>
+__device__ __forceinline__ V3T<M> vertex_force_factors(const CellViewT<M>& c, const TypeDev& T, int k, M vforce,
+                                                       const M* bx, const M* by, const M* bz, const M* vx, const M* vy,
+                                                       const M* vz, bool visc) {
+  const RingOf ring(T, k);
+  const uint4 rq = T.cring[k], tid = T.rid[2 * k], eid = T.rid[2 * k + 1];
+  const V3T<M> xk = c.pos(k);
+  M F0, F1, F2;
+  TriangleSum<M> sum;
+#pragma unroll 1
+  for (int j = 0; j < ring.nr; ++j) {
+    const V3T<M> a = c.pos(ring_entry(rq, j)) - xk;
+    const V3T<M> b = c.pos(ring_entry(rq, j + 1 < ring.nr ? j + 1 : 0)) - xk;
+    sum.add(a, b, triangle_factor(c, T, ring_entry(tid, j)));
+  }
+  sum.force(T, vforce, F0, F1, F2);
+  gather_bending<M>(ring, k, bx, by, bz, F0, F1, F2);
+#pragma unroll 1
+  for (int j = 0; j < ring.nr; ++j) {
+    const V3T<M> d = c.pos(ring_entry(rq, j)) - xk;
+    const M f = edge_factor(c, T, ring_entry(eid, j), vx, vy, vz, visc);
+    F0 += d.x * f;
+    F1 += d.y * f;
+    F2 += d.z * f;
+  }
+  inner_forces<MODEL, M>(c, T, k, F0, F1, F2);
+  return {F0, F1, F2};
 }
 
 // Force on vertex k of one cell: every term gathered in the reference's order
