@@ -26,6 +26,9 @@
 //   cu = c_i.u, cF = c_i.F, A = omega (rhoBar - 3/2 rho u^2) - 3 mu u.F,
 //   B = 3 omega rho, C = 9/2 omega rho, D = 3 mu, E = 9 mu,
 // split into even and odd parts over each opposite pair (i, i+9).
+//
+// Compiled once per precision (HC_REAL, float or double), with other rules for
+// fusing multiply-adds (Makefile).
 #include <utility>
 
 #include "hc_d3q19.h"
@@ -714,8 +717,7 @@ hipError_t launch_lees_edwards(hipStream_t s, R* f, const uint8_t* type, const L
   template hipError_t launch_lees_edwards<R>(hipStream_t, R*, const uint8_t*, const LatticeDev&, int,             \
                                              const CollideArgs&, double, double, double, R*);                  \
   template hipError_t launch_collide_multi<R>(hipStream_t, const LatCase*, int, uint32_t, int, bool, bool);
-HC_INSTANTIATE(float)
-HC_INSTANTIATE(double)
+HC_INSTANTIATE(HC_REAL)
 #undef HC_INSTANTIATE
 
 }  // namespace hcg

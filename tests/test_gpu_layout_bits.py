@@ -1,5 +1,5 @@
 """With the exact spread a cell ends in the same bits however its launch lays out its positions: staged, in LDS only, or
-in global memory beside many red cells and in the persistent launch."""
+in global memory beside many red cells and in the persistent launch; alone and in a batch."""
 import numpy as np
 import pytest
 
@@ -59,11 +59,15 @@ def _sim(monkeypatch, frequency, mixed):
 # 642: staged, but for the persistent launch
 @pytest.mark.parametrize("frequency", [8, 12, 14])
 def test_launches_agree(monkeypatch, frequency):
+    import hemocell_amd as hc
     out = []
-    for how in ("alone", "in LDS", "persistent"):
+    for how in ("alone", "in LDS", "persistent", "batch"):
         monkeypatch.setenv("HC_SIDE_GPOS", "0" if how == "in LDS" else "1")
         s = _sim(monkeypatch, frequency, "1" if how == "persistent" else "0")
-        s.step(6)
+        if how == "batch":
+            hc.step_batch([s], 6)
+        else:
+            s.step(6)
         out.append(s.vertices() + (s.populations(),))
         s.close()
     for other in out[1:]:
