@@ -6,6 +6,7 @@
 
 #include "hc_d3q19.h"
 #include "hc_launch.h"
+#include "hc_wrap.h"
 
 namespace hcg {
 namespace {
@@ -33,14 +34,6 @@ struct SupportT {
   int lo[3];  // unwrapped coordinates of the slot-0 node
 };
 using Support = SupportT<double>;
-
-// Coordinate of node fl (an integer, |fl| < 2^53) on a periodic axis of size n.
-__device__ __forceinline__ int wrap_node(double fl, int n) {
-  double m = fl - (double)n * floor(fl / (double)n);
-  if (m < 0.0) m += (double)n;
-  if (m >= (double)n) m -= (double)n;
-  return (int)m;
-}
 
 // Node indices and normalised weights from the low corner n0 and the hat values
 // q of each axis.  A support inside the domain (all but the vertices at a domain
