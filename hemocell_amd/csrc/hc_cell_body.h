@@ -865,8 +865,11 @@ hipError_t launch_cell_step_mixed(hipStream_t s, const VertexDev& V, const TypeD
     visc[t] = (h_types[t].model != HC_MODEL_RBC) || (h_types[t].eta_m != 0.0);
   }
   MixedArgs A{};
-  const size_t dyn = mixed_lds_plan(ntypes, model, nv, visc, sizeof(MechT<R, true, false>), (size_t)box_bytes,
-                                    (size_t)lds_device, st, A.box_nodes);
+  size_t dyn = 0;
+  for (size_t box : {(size_t)box_bytes, std::min((size_t)box_bytes, kLeastBox)})
+    if (dyn == 0)
+      dyn = mixed_lds_plan(ntypes, model, nv, visc, sizeof(MechT<R, true, false>), box, (size_t)lds_device, st,
+                           A.box_nodes);
   if (dyn == 0) return hipErrorInvalidConfiguration;
   for (int t = 0; t < ntypes; ++t) A.flags[t] = flags[t];
   hipError_t e = launch_fill_zero<float>(s, reinterpret_cast<float*>(head), 1);
@@ -883,8 +886,8 @@ template <typename R>
 bool cell_step_all_plan(const TypeDev& T, int box_bytes, int lds_device, int* box_nodes, size_t* dyn) {
   static const size_t st = static_lds(k_cell_step_all<R>);
   const bool visc = (T.model != HC_MODEL_RBC) || (T.eta_m != 0.0);
-  const CellLdsPlan p = cell_lds_plan(T.model, T.nv, visc, sizeof(MechT<R, true, false>), (size_t)box_bytes,
-                                      (size_t)lds_device, st, st, st, false);
+  const CellLdsPlan p = cell_lds_layout(T.model, T.nv, visc, sizeof(MechT<R, true, false>), (size_t)box_bytes,
+                                        (size_t)lds_device, st, st, st, POS_LDS);
   if (!p.ok || !p.staged) return false;
   *box_nodes = p.box_nodes;
   *dyn = std::max(*dyn, p.dyn);

@@ -74,13 +74,28 @@ inline CellLdsPlan cell_lds_plan(int model, int nv, bool visc, size_t psize, siz
 // as float offsets, the others as doubles), in LDS as doubles, or in global memory.
 enum CellPositions { POS_LDS = 0, POS_LDS_DOUBLE = 1, POS_GLOBAL = 2 };
 
-// cell_lds_plan for a launch that may ask for positions as doubles, which with float
-// offsets in the staged layout (psize 4) leaves the plain one.
+// The spread scratch a layout is chosen for.
+constexpr size_t kLeastBox = 12288;
+
+// The layout of a launch.  Chosen for kLeastBox, so that a mesh keeps its layout, and
+// with it the precision of its mechanics (the staged layout holds float offsets in
+// the FP32-shifted form), however much scratch a launch asks for, and a large mesh is
+// not refused for it (from 45953 vertices on with 69632 bytes); the rest is granted
+// as far as there is room.  Positions as doubles: with float offsets in the staged
+// layout (psize 4) that leaves the plain one.
 inline CellLdsPlan cell_lds_layout(int model, int nv, bool visc, size_t psize, size_t box_bytes, size_t lds_device,
                                    size_t st_staged, size_t st_plain, size_t st_gpos, CellPositions pos) {
   const bool plain = pos == POS_LDS_DOUBLE && psize != sizeof(double);
-  return cell_lds_plan(model, nv, visc, psize, box_bytes, lds_device, plain ? lds_device : st_staged, st_plain,
-                       st_gpos, pos == POS_GLOBAL);
+  CellLdsPlan p = cell_lds_plan(model, nv, visc, psize, std::min(box_bytes, kLeastBox), lds_device,
+                                plain ? lds_device : st_staged, st_plain, st_gpos, pos == POS_GLOBAL);
+  if (p.ok && box_bytes > p.region) {
+    const size_t st = p.staged ? st_staged : (pos == POS_GLOBAL ? st_gpos : st_plain);
+    const size_t room = (lds_device - st - kLdsMargin - p.fixed - p.lists) & ~(size_t)15;
+    p.region = std::max(p.region, std::min(box_bytes, room));
+    p.dyn = p.fixed + p.region + p.lists;
+    p.box_nodes = (int)(p.region / (3 * sizeof(double)));
+  }
+  return p;
 }
 
 // The persistent mixed launch: one dynamic size for every type (staged RBC and
