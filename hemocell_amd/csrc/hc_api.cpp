@@ -94,7 +94,8 @@ struct hc_ctx {
   int lds_limit = 65536;        // dynamic LDS per workgroup available on the device
   int lds_device = 65536;       // LDS per workgroup of the device (static + dynamic)
   bool spread_per_cell = true;  // LDS-staged spread (false: one thread per vertex, global atomics)
-  int spread_lds = 0;           // LDS box budget in bytes (0: default per precision)
+  int spread_lds = 0;           // spread scratch of the cell kernels in bytes (0: spread_box_bytes)
+  int alone_lds = 0;            // LDS box budget of the spread by itself in bytes (0: 65536)
   bool side_gpos = true;        // large-cell side types read positions from global memory
   int cell_block = 256;         // threads per RBC cell in the fused vertex kernel
   int wbc_block = 1024;         // threads per WBC cell (falls back when the LDS does not fit)
@@ -847,7 +848,7 @@ hc_status do_spread(hc_ctx* ctx) {
   if (ctx->n_extra > 0) HC_TRY(launch_add_extra_force(ctx->stream, vdev(ctx), ctx->d_extra_ids, ctx->d_extra_f, ctx->n_extra), "extra force");
   if (ctx->spread_per_cell) {
     // LDS budget (a box of doubles): room for the support box of an aligned RBC
-    const int want = ctx->spread_lds > 0 ? ctx->spread_lds : 65536;
+    const int want = ctx->alone_lds > 0 ? ctx->alone_lds : 65536;
     HC_TRY(launch_spread_cells<R>(ctx->stream, vdev(ctx), (R*)ctx->Fibm[ctx->cur], ctx->type, ctx->L, ctx->d_cell_base,
                                   ctx->d_cell_nv, (int)ctx->cell_base.size(), ctx->f_limit, rep_mask(ctx),
                                   std::min(want, ctx->lds_limit)),
@@ -1395,8 +1396,12 @@ hc_status batch_impl(hc_ctx* const* cs, int n, int nsteps) {
 
 // Autotuner: times real steps of this context (HIP events on its stream, steps
 // launched eagerly) for each value of one parameter at a time -- the spread
-// box, the threads per RBC cell, the side types' layout, the threads per WBC
-// cell -- and keeps the fastest.  The steps advance the simulation as any other.
+// scratch, the threads per RBC cell, the side types' layout, the threads per WBC
+// cell -- and keeps the fastest.  The first value of each is what the context runs
+// with, 0 the rule by model and number of cells (spread_box_bytes, cell_threads);
+// another one replaces it when it is faster by more than the trials differ, 1%: a
+// lone RBC lost its one-pass spread to the fastest of the others (46 -> 52 us per
+// step).  The steps advance the simulation as any other.
 template <typename R>
 hc_status autotune_impl(hc_ctx* ctx, int steps, std::string& report) {
   const bool graphs = ctx->use_graphs;
@@ -1436,18 +1441,24 @@ hc_status autotune_impl(hc_ctx* ctx, int steps, std::string& report) {
   // the per-type launches side by side first, then the one persistent launch of
   // all types against them, and its workgroups per compute unit when it wins
   const bool queue = ctx->d_queue && ntypes > 1;
+  const int block0 = ctx->cell_block;
+  const bool env0 = ctx->cell_block_env;
   std::vector<Param> params = {
-      {"spread_box_bytes", {8192, 12288, 16384, 20480, 24576}, [&](int v) { ctx->spread_lds = v; },
+      {"spread_box_bytes", {ctx->spread_lds, 8192, 12288, 16384, 20480, 24576}, [&](int v) { ctx->spread_lds = v; },
        [] { return true; }},
-      {"rbc_threads", {256, 512, 1024}, [&](int v) { ctx->cell_block = v; ctx->cell_block_env = true; },
+      {"rbc_threads", {env0 ? block0 : 0, 256, 512, 1024},
+       [&](int v) {
+         ctx->cell_block = v ? v : block0;
+         ctx->cell_block_env = v != 0;
+       },
        [&] { return has_rbc; }},
-      {"side_positions_global", {1, 0}, [&](int v) { ctx->side_gpos = v != 0; },
+      {"side_positions_global", {ctx->side_gpos, !ctx->side_gpos}, [&](int v) { ctx->side_gpos = v != 0; },
        [&] { return ntypes > 1 && big_side; }},
       // a side WBC with positions in global memory always runs 256 threads
-      {"wbc_threads", {256, 512, 1024}, [&](int v) { ctx->wbc_block = v; },
+      {"wbc_threads", {ctx->wbc_block, 256, 512, 1024}, [&](int v) { ctx->wbc_block = v; },
        [&] { return has_wbc && !(ctx->side_gpos && ntypes > 1 && big_side); }},
-      {"persistent_launch", {0, 1}, [&](int v) { ctx->mixed = v != 0; }, [&] { return queue; }},
-      {"persistent_workgroups_per_cu", {4, 8, 16}, [&](int v) { ctx->mixed_per_cu = v; },
+      {"persistent_launch", {ctx->mixed, !ctx->mixed}, [&](int v) { ctx->mixed = v != 0; }, [&] { return queue; }},
+      {"persistent_workgroups_per_cu", {ctx->mixed_per_cu, 4, 8, 16}, [&](int v) { ctx->mixed_per_cu = v; },
        [&] { return ctx->mixed; }},
   };
   std::ostringstream out;
@@ -1455,16 +1466,20 @@ hc_status autotune_impl(hc_ctx* ctx, int steps, std::string& report) {
   bool first_param = true;
   for (auto& p : params) {
     if (!p.on() || s != HC_OK) continue;
-    int best = p.values[0];
+    const int first = p.values[0];
+    int best = first;
     double best_ms = 1e300;
     out << (first_param ? "" : ", ") << "\"" << p.name << "\": {";
     first_param = false;
     for (size_t k = 0; k < p.values.size(); ++k) {
+      if (k && p.values[k] == first) continue;
       p.set(p.values[k]);
       double ms = 0;
       if ((s = trial(ms)) != HC_OK) break;
       out << (k ? ", " : "") << "\"" << p.values[k] << "\": " << ms;
-      if (ms < best_ms) {
+      if (k == 0) {
+        best_ms = 0.99 * ms;
+      } else if (ms < best_ms) {
         best_ms = ms;
         best = p.values[k];
       }
@@ -1602,7 +1617,7 @@ hc_status hc_create(int device, hc_ctx** out) {
   const char* gr = std::getenv("HC_GRAPH");  // 0: launch every step eagerly
   if (gr && std::string(gr) == "0") ctx->use_graphs = false;
   const char* sl = std::getenv("HC_SPREAD_LDS");  // tuning: LDS bytes of the per-cell box
-  if (sl) ctx->spread_lds = std::atoi(sl);
+  if (sl) ctx->spread_lds = ctx->alone_lds = std::atoi(sl);
   const char* sg = std::getenv("HC_SIDE_GPOS");  // tuning: 0 stages every type's positions in LDS
   if (sg) ctx->side_gpos = std::atoi(sg) != 0;
   const char* mx = std::getenv("HC_MIXED");  // tuning: 1 runs every cell type in one persistent launch

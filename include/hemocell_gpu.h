@@ -264,7 +264,9 @@ int hc_busy(hc_ctx* ctx);
 int64_t hc_iteration(const hc_ctx* ctx);
 /* Picks the launch shapes of the per-cell kernels for this context's mesh mix (spread box
  * bytes, threads per RBC cell, side types' position layout, threads per WBC cell) by
- * timing steps_per_trial real steps per candidate, one parameter at a time; the steps
+ * timing steps_per_trial real steps per candidate, one parameter at a time; the shapes
+ * the context runs with are the first candidates (0: chosen by model and number of cells)
+ * and stay unless another is faster by more than 1%.  The steps
  * advance the simulation.  report (may be NULL) receives the timings and choices as JSON.
  * No counterpart in the reference (its kernels have no launch shape to choose). */
 hc_status hc_autotune(hc_ctx* ctx, int steps_per_trial, char* report, int report_len);
