@@ -269,7 +269,7 @@ __device__ __forceinline__ void cell_step_body(const VertexDev& V, const TypeDev
         for (int a = 0; a < 3; ++a) {
           const double fl = floor(p[a] + 0.5);
           if (fl >= 0.0 && fl < (double)dims[a]) wc[a] = (int)fl;
-          else if (L.periodic[a]) wc[a] = wrap_node(fl, dims[a]);
+          else if (L.periodic[a]) wc[a] = wrap_far(fl, dims[a]);
           else out = true;
         }
         if (!out && type[(uint32_t)wc[2] + (uint32_t)L.nz * ((uint32_t)wc[1] + (uint32_t)L.ny * (uint32_t)wc[0])] !=

@@ -4,4 +4,5 @@
 
 extern "C" {
 int wrap_node(double fl, int n) { return hcg::wrap_node(fl, n); }
+int wrap_far(double fl, int n) { return hcg::wrap_far(fl, n); }
 }

@@ -17,7 +17,8 @@ def lib(tmp_path_factory):
     subprocess.check_call(["g++", "-O1", "-std=c++17", "-ffp-contract=off", "-shared", "-fPIC", "-o", out,
                            os.path.join(HERE, "native", "wrap_shim.cpp")])
     L = ctypes.CDLL(out)
-    L.wrap_node.argtypes, L.wrap_node.restype = [ctypes.c_double, ctypes.c_int], ctypes.c_int
+    for f in (L.wrap_node, L.wrap_far):
+        f.argtypes, f.restype = [ctypes.c_double, ctypes.c_int], ctypes.c_int
     return L
 
 
@@ -28,6 +29,7 @@ def test_any_finite_node(lib, n):
     far = [math.floor(10.0 ** rng.uniform(0, 308)) for _ in range(3000)]
     for fl in edges + far + [1.7976931348623157e308]:
         for x in (float(fl), -float(fl)):
-            assert lib.wrap_node(x, n) == int(x) % n, (x, n)
+            assert lib.wrap_far(x, n) == int(x) % n, (x, n)
+            assert abs(x) > 2.0 ** 52 or lib.wrap_node(x, n) == int(x) % n, (x, n)
     for x in (math.inf, -math.inf, math.nan):
-        lib.wrap_node(x, n)  # no node, but it returns
+        lib.wrap_far(x, n)  # no node, but it returns
