@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "hc_launch.h"
+#include "hc_stage.h"
 
 using namespace hcg;
 
@@ -170,12 +171,6 @@ struct hc_ctx {
   int32_t* d_vcell = nullptr;
   unsigned long long* d_wall_hits = nullptr;
   unsigned int* d_flag = nullptr;
-  // read-back staging: per reader two pinned slots of stage_cap bytes that the
-  // read-back kernels fill in turn, made on the first read-back (of the size that
-  // takes that reader) and kept
-  void* h_stage[2 * kReaders] = {};
-  size_t stage_cap[kReaders] = {};
-  hipEvent_t stage_ev[2 * kReaders] = {};
   Prof prof;
 };
 
@@ -266,46 +261,51 @@ struct DeviceScope {
 };
 
 // bytes of one read-back slot at most: a chunk's launch and wait (~10 us) stay below
-// its 20 us on the link, the host's copy of it hits its caches, and pinning the two
-// slots costs a context's first read-back little (with 4 MB slots 3 ms of it)
+// its 20 us on the link, the host's copy of it hits its caches, and pinning it costs
+// little (with two slots of 4 MB a first read-back 3 ms of it)
 constexpr size_t kStageBytes = size_t(1) << 20;
 
-// two pinned slots of at least `bytes` each (at most kStageBytes) for reader `t`
-hc_status ensure_stage(hc_ctx* ctx, size_t bytes, int t = 0) {
-  for (int k = 2 * t; k < 2 * t + 2; ++k)
-    if (!ctx->stage_ev[k]) HC_TRY(hipEventCreateWithFlags(&ctx->stage_ev[k], hipEventDisableTiming), "hipEventCreate");
-  if (ctx->stage_cap[t] >= bytes) return HC_OK;
-  size_t cap = 65536;
-  while (cap < bytes) cap *= 2;
-  for (int k = 2 * t; k < 2 * t + 2; ++k) {
-    if (ctx->h_stage[k]) hipHostFree(ctx->h_stage[k]);
-    ctx->h_stage[k] = nullptr;
+// Pinned slots of the device's pool for one call, returned at its end.
+struct Staging {
+  hc_ctx* ctx;
+  StageSlot slot[2 * kReaders];
+  bool failed = false;  // something may still write to them
+  explicit Staging(hc_ctx* c) : ctx(c) {}
+  Staging(const Staging&) = delete;
+  ~Staging() {
+    if (failed) (void)hipStreamSynchronize(ctx->stream);
+    for (const StageSlot& s : slot)
+      if (s.p) StagePool::of(ctx->device).give(s);
   }
-  ctx->stage_cap[t] = 0;
-  for (int k = 2 * t; k < 2 * t + 2; ++k)
-    if (hipHostMalloc(&ctx->h_stage[k], cap, hipHostMallocDefault) != hipSuccess) {
-      (void)hipGetLastError();
-      return fail(ctx, HC_OOM, "pinned host allocation of the read-back staging failed");
-    }
-  ctx->stage_cap[t] = cap;
-  return HC_OK;
-}
+  // slots first..first+n-1, of at least `bytes` (at most kStageBytes) each
+  bool take(int first, int n, size_t bytes) {
+    for (int k = first; k < first + n; ++k)
+      if (!StagePool::of(ctx->device).take(bytes, slot[k])) return false;
+    return true;
+  }
+  hc_status take(size_t bytes, int n = 1) {
+    return take(0, n, bytes) ? HC_OK
+                             : fail(ctx, HC_OOM, "pinned host allocation of the read-back staging failed");
+  }
+};
 
-// the items begin..end of staged_read through the slots of reader `t`
+// the items begin..end of staged_read through the two slots at `slots` (one chunk: the
+// first alone)
 template <typename Launch, typename Take>
-hipError_t staged_range(hc_ctx* ctx, int t, int64_t begin, int64_t end, int64_t chunk, Launch& launch, Take& take) {
+hipError_t staged_range(hc_ctx* ctx, const StageSlot* slots, int64_t begin, int64_t end, int64_t chunk, Launch& launch,
+                        Take& take) {
   int64_t before = -1, nbefore = 0;
-  int slot = 2 * t;
+  int slot = 0;
   for (int64_t first = begin; first < end || before >= 0; first += chunk) {
     const int64_t n = first < end ? std::min(chunk, end - first) : 0;
     hipError_t e;
     if (n > 0) {
-      if ((e = launch(first, n, ctx->h_stage[slot])) != hipSuccess) return e;
-      if ((e = hipEventRecord(ctx->stage_ev[slot], ctx->stream)) != hipSuccess) return e;
+      if ((e = launch(first, n, slots[slot].p)) != hipSuccess) return e;
+      if ((e = hipEventRecord(slots[slot].ev, ctx->stream)) != hipSuccess) return e;
     }
     if (before >= 0) {
-      if ((e = hipEventSynchronize(ctx->stage_ev[slot ^ 1])) != hipSuccess) return e;
-      take(before, nbefore, ctx->h_stage[slot ^ 1]);
+      if ((e = hipEventSynchronize(slots[slot ^ 1].ev)) != hipSuccess) return e;
+      take(before, nbefore, slots[slot ^ 1].p);
     }
     before = n > 0 ? first : -1;
     nbefore = n;
@@ -335,14 +335,16 @@ hc_status staged_read(hc_ctx* ctx, int64_t items, size_t item_bytes, const char*
     readers = (int)std::min<unsigned>(kReaders, std::max(1u, std::thread::hardware_concurrency() / 2));
   const size_t slot_bytes = readers > 1 ? kStageBytes / 2 : kStageBytes;
   const int64_t chunk = std::min(items, std::max<int64_t>(1, (int64_t)(slot_bytes / item_bytes)));
-  hc_status s = ensure_stage(ctx, (size_t)chunk * item_bytes);
+  Staging staging(ctx);
+  const hc_status s = staging.take((size_t)chunk * item_bytes, items > chunk ? 2 : 1);
   if (s != HC_OK) return s;
   for (int t = 1; t < readers; ++t)
-    if (ensure_stage(ctx, (size_t)chunk * item_bytes, t) != HC_OK) readers = t;  // fewer readers do
+    if (!staging.take(2 * t, 2, (size_t)chunk * item_bytes)) readers = t;  // fewer readers do
   const int64_t share = (items + readers - 1) / readers;
   hipError_t e[kReaders] = {};
   auto read = [&](int t) {
-    e[t] = staged_range(ctx, t, std::min(items, t * share), std::min(items, (t + 1) * share), chunk, launch, take);
+    e[t] = staged_range(ctx, staging.slot + 2 * t, std::min(items, t * share), std::min(items, (t + 1) * share), chunk,
+                        launch, take);
   };
   std::thread threads[kReaders];
   for (int t = 1; t < readers; ++t) {
@@ -359,6 +361,7 @@ hc_status staged_read(hc_ctx* ctx, int64_t items, size_t item_bytes, const char*
     if (threads[t].joinable()) threads[t].join();
     else read(t);
   }
+  for (int t = 0; t < readers; ++t) staging.failed = staging.failed || e[t] != hipSuccess;
   for (int t = 0; t < readers; ++t) HC_TRY(e[t], what);
   return HC_OK;
 }
@@ -1510,9 +1513,10 @@ template <typename R>
 static hc_status fluid_stats(hc_ctx* ctx, int what, double* out) {
   const DeviceScope on(ctx->device);
   const int nb = (int)std::min<int64_t>(4096, (ctx->L.N + 255) / 256);
-  hc_status s = ensure_stage(ctx, sizeof(double) * 4 * nb);
+  Staging staging(ctx);
+  const hc_status s = staging.take(sizeof(double) * 4 * nb);
   if (s != HC_OK) return s;
-  double* const h = (double*)ctx->h_stage[0];  // the blocks' partials, written by the kernel
+  double* const h = (double*)staging.slot[0].p;  // the blocks' partials, written by the kernel
   R* Fs = nullptr;
   CollideArgs a{};
   a.omega = 1.0 / ctx->tau;
@@ -1534,6 +1538,7 @@ static hc_status fluid_stats(hc_ctx* ctx, int what, double* out) {
   if (e == hipSuccess)
     e = launch_fluid_stats<R>(ctx->stream, (const R*)ctx->f, Fc, ctx->type, ctx->L, ctx->phase, a, Fs, what, h, nb);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+  staging.failed = e != hipSuccess;
   if (e != hipSuccess) return hipfail(ctx, e, "fluid statistics");
   double mn = INFINITY, mx = -INFINITY, sum = 0.0, cnt = 0.0;
   for (int b = 0; b < nb; ++b) {
@@ -1624,6 +1629,7 @@ hc_status hc_create(int device, hc_ctx** out) {
   if (mx) ctx->mixed = std::atoi(mx) != 0;
   const char* mp = std::getenv("HC_MIXED_PER_CU");  // tuning: its workgroups per compute unit
   if (mp && std::atoi(mp) > 0) ctx->mixed_per_cu = std::atoi(mp);
+  StagePool::of(device).open();
   *out = ctx;
   return HC_OK;
 }
@@ -1656,11 +1662,8 @@ void hc_destroy(hc_ctx* ctx) {
     if (ctx->batch_slot_ev[k]) hipEventDestroy(ctx->batch_slot_ev[k]);
     if (ctx->h_batch[k]) hipHostFree(ctx->h_batch[k]);
   }
-  for (int k = 0; k < 2 * kReaders; ++k) {
-    if (ctx->h_stage[k]) hipHostFree(ctx->h_stage[k]);
-    if (ctx->stage_ev[k]) hipEventDestroy(ctx->stage_ev[k]);
-  }
   hipStreamDestroy(ctx->stream);
+  StagePool::of(ctx->device).close();
   delete ctx;
 }
 
@@ -2538,8 +2541,9 @@ hc_status hc_get_cell_stats(hc_ctx* ctx, double* volume, double* area, double* c
   const size_t bytes = sizeof(double) * NQ * nc;
   const bool direct = bytes <= kStageBytes;
   double* d = nullptr;
-  if ((s = direct ? ensure_stage(ctx, bytes) : dalloc(ctx, (void**)&d, bytes, "cell statistics")) != HC_OK) return s;
-  if (direct) d = (double*)ctx->h_stage[0];
+  Staging staging(ctx);
+  if ((s = direct ? staging.take(bytes) : dalloc(ctx, (void**)&d, bytes, "cell statistics")) != HC_OK) return s;
+  if (direct) d = (double*)staging.slot[0].p;
   hipError_t e = hipSuccess;
   for (auto& tp : ctx->types)
     if (e == hipSuccess && tp->ncells)
@@ -2548,6 +2552,7 @@ hc_status hc_get_cell_stats(hc_ctx* ctx, double* volume, double* area, double* c
   if (e == hipSuccess && !direct) e = hipMemcpyAsync(copy.data(), d, bytes, hipMemcpyDeviceToHost, ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (!direct) hipFree(d);
+  staging.failed = e != hipSuccess;
   if (e != hipSuccess) return hipfail(ctx, e, "cell statistics");
   const double* const h = direct ? d : copy.data();
   for (int c = 0; c < nc; ++c) {
