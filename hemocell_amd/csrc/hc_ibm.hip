@@ -321,8 +321,10 @@ __global__ __launch_bounds__(BS) void k_spread_cells(VertexDev V, R* __restrict_
   if (tid == 0) write_box(V.box ? V.box + kBoxInts * (int64_t)cell : nullptr, bmin, bmax, bad != 0);
   const int o0 = bmin[0], o1 = bmin[1], o2 = bmin[2];
   const int s0 = bmax[0] - bmin[0] + 2, s1 = bmax[1] - bmin[1] + 2, s2 = bmax[2] - bmin[2] + 2;
-  const int64_t total = (int64_t)s0 * s1 * s2;
-  const bool direct = bad || total > lds_nodes || s0 <= 0;
+  // each size by itself first: the product of three up to 2e9 would not fit
+  const bool small = !bad && s0 > 0 && s0 <= lds_nodes && s1 <= lds_nodes && s2 <= lds_nodes;
+  const int64_t total = small ? (int64_t)s0 * s1 * s2 : 0;
+  const bool direct = !small || total > lds_nodes;
   if (!direct)
     for (int64_t e = tid; e < 3 * total; e += BS) box[e] = 0.0;
   __syncthreads();

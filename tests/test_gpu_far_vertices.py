@@ -37,3 +37,33 @@ def test_wall_contact(monkeypatch, far, precision):
         s.close()
     assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
     assert 0 < out[0][1] < len(k)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+# sizes of the support box whose product is 0 or negative in 64 bits
+@pytest.mark.parametrize("size", [(2 ** 22, 2 ** 22, 2 ** 22), (2 ** 21, 2 ** 21, 2 ** 21), (2 ** 23, 2 ** 22, 2 ** 23),
+                                  (2 ** 29, 2 ** 29, 2 ** 29)])
+def test_spread_of_a_cell_across_the_axes(monkeypatch, size, precision):
+    """A periodic box, a cell whose vertices lie millions of nodes apart: its spread by itself adds the same force as the
+    spread by vertex."""
+    import hemocell_amd as hc
+    u = cases.units()
+    model, v, t, p, inner = cases.mesh("RBC", u, hc.build_mesh)
+    out = []
+    for spread in ("vertex", "cell"):
+        monkeypatch.setenv("HC_SPREAD", spread)
+        s = hc.Simulation(0)
+        s.lattice_init(31, 24, 37, u.tau, precision=precision)
+        s.init_equilibrium(1.0, [0, 0, 0])
+        s.set_force_limit(u.f_limit)
+        s.add_cells(s.add_cell_type(model, v, t, p, inner), cases.place(v, (15, 12, 18))[None])
+        x = s.vertices()[0]
+        x[5] = (3.25, 4.5, 5.75)
+        x[9] = x[5] + np.array(size) - 2
+        x = np.clip(x, x[5], x[9])
+        f = np.random.default_rng(3).uniform(-1e-5, 1e-5, x.shape)
+        s.set_vertices(x=x, f=f)
+        s.stage("spread")
+        out.append(s.force_field())
+        s.close()
+    assert np.abs(out[0]).max() > 0 and cases.rel_l2(out[1], out[0]) < (1e-6 if precision else 1e-14)
