@@ -712,9 +712,9 @@ hc_status do_visc_membrane(hc_ctx* ctx, const double* xold) {
 // per support node in one pass.  An RBC touches ~1290 nodes in at most 306 rows, a
 // platelet at most 97 in 36, the 8 um WBC 2210 in 324.
 // Many cells: an RBC's spread takes two passes, so that five FP32 (four FP64)
-// workgroups share a compute unit's 160 KB: 15.5k RBC, FP32 step 3.12 ms with
-// 18432 bytes (three passes), 3.08 with 21504, 3.31 with 24576 (four workgroups),
-// 3.48 with 40960 (one pass, three workgroups).
+// workgroups share a compute unit's 160 KB.  15.5k RBC, ms per step in FP32 / FP64:
+// 18432 bytes (three passes) 3.05 / 5.59, 20480 and 21504 3.00 / 5.48, 24576 (one
+// workgroup fewer) 3.05 / 5.61, 40960 (one pass) 3.11 / 5.86.
 // Few cells, which occupy a compute unit alone: everything in one pass.
 int spread_box_bytes(const hc_ctx* c, int model, bool few) {
   // a platelet's nodes all fit, and a larger region only keeps its workgroups from

@@ -18,8 +18,9 @@
 // kernel; per-vertex bending forces and velocities too when they fit.
 //
 // Instantiated by hc_cell_f64.hip (FP64, compiled without contracting
-// multiply-adds so the FP64 form follows the oracle's operation order) and
-// hc_cell_f32.hip (the FP32-shifted form, which may fuse them).
+// multiply-adds, so that every layout and launch rounds alike; its red and white
+// cells sum around a vertex's ring, not in the oracle's order) and hc_cell_f32.hip
+// (the FP32-shifted form, which may fuse them).
 #pragma once
 #include <algorithm>
 #include <type_traits>
@@ -785,10 +786,9 @@ static size_t static_lds(K kernel) {
 }
 
 // Lay out the dynamic LDS of one cell type for block size B and launch: staged
-// (positions, velocities and a region shared by bending forces and the box) when
-// it fits beside the kernel's static LDS, else positions plus as much box as
-// fits; with gpos only the box.  The spread's vertex list (2 bytes per vertex)
-// follows the region.
+// (positions, velocities and a region shared by the mechanics and the spread's
+// scratch) when it fits beside the kernel's static LDS, else positions plus as much
+// scratch as fits; with positions in global memory only the scratch.
 template <typename R, int M, int B>
 static hipError_t launch_cell(hipStream_t s, const VertexDev& V, const TypeDev& T, const int32_t* cells, int ncells,
                               const int64_t* cell_base, const R* uf, const uint8_t* type, const LatticeDev& L, R* Fnext,

@@ -6,11 +6,11 @@
 //   fixed   positions (3 nv scalars) and, staged with a viscous membrane, the
 //           vertex velocities (3 nv more), rounded up to 16 bytes; in the plain
 //           layout 3 nv doubles; nothing when the positions stay in global memory;
-//   region  the bending forces of the mechanics (staged, 3 nv scalars; platelets:
-//           the terms of each edge, 6 scalars) and then the spread box (3 doubles
-//           per node) over the same bytes;
-//   lists   the spread's bucketed vertex list (2 bytes per vertex), which the
-//           kernel places right after the box's last node.
+//   region  the mechanics' forces and factors (staged: 3 nv scalars for the bending
+//           forces, and the factors of triangles and edges beside them where it is
+//           large enough; platelets: the terms of each edge, 6 scalars) and then the
+//           spread's scratch (row masks and node sums) over the same bytes;
+//   lists   2 bytes per vertex, part of the spread's scratch.
 #pragma once
 #include <algorithm>
 #include <cstddef>
@@ -42,7 +42,7 @@ struct CellLdsPlan {
   bool ok;        // fits beside the kernel's static LDS within the workgroup limit
   bool staged;    // the layout the launch uses (staged may fall back to plain)
   size_t fixed, region, lists, dyn;
-  int box_nodes;  // spread box nodes: 3 doubles each, within the region
+  int box_nodes;  // of 24 bytes each, within the region
 };
 
 // One cell type's layout for a launch of the per-type kernel.  st_* are the

@@ -875,18 +875,7 @@ __device__ __forceinline__ double volume_partial(const CellViewT<M>& c, const Ty
   // spacings from the origin (FP64 whatever the position type)
   const V3T<M> rm = c.pos(0);
   const D3 r = {(double)rm.x, (double)rm.y, (double)rm.z};
-  for (int t = tid; t < T.nt; t += BS) {
-    const V3T<M> a = c.pos(T.tri[3 * t]), b = c.pos(T.tri[3 * t + 1]), e = c.pos(T.tri[3 * t + 2]);
-    const D3 v0 = D3{(double)a.x, (double)a.y, (double)a.z} - r, v1 = D3{(double)b.x, (double)b.y, (double)b.z} - r,
-             v2 = D3{(double)e.x, (double)e.y, (double)e.z} - r;
-    const double v210 = v2.x * v1.y * v0.z;
-    const double v120 = v1.x * v2.y * v0.z;
-    const double v201 = v2.x * v0.y * v1.z;
-    const double v021 = v0.x * v2.y * v1.z;
-    const double v102 = v1.x * v0.y * v2.z;
-    const double v012 = v0.x * v1.y * v2.z;
-    part += (-v210 + v120 + v201 - v021 - v102 + v012);
-  }
+  for (int t = tid; t < T.nt; t += BS) part += volume_term(c, T, t, r);
   return part;
 }
 

@@ -40,8 +40,10 @@ typedef enum {
 
 typedef enum {
   HC_FP64 = 0,          /* FP64 populations and collision: the correctness mode */
-  HC_FP32_SHIFTED = 1   /* FP32 populations (f_i - t_i) and FP32 collision; vertex
-                           state, IBM weights and mechanics stay FP64 */
+  HC_FP32_SHIFTED = 1   /* FP32 populations (f_i - t_i), collision, IBM weights and, of
+                           cells staged in LDS, membrane forces; vertex state and
+                           volumes stay FP64, and so do the forces of a large cell type
+                           (over 1365 vertices) beside a main one */
 } hc_precision;
 
 /* Node types of the lattice mask (one uint8 per node). */
@@ -142,7 +144,8 @@ hc_status hc_set_force_limit(hc_ctx* ctx, double f_limit);
  * on != 0 (FP64 form only; needs a force limit, and the lattice), every force contribution
  * is rounded to a multiple of 2^(e-49), 2^e <= f_limit < 2^(e+1), before it is added: the
  * sums are then exact up to 8 force limits per node, so repeated runs, a run alone or in a
- * batch, and a run resumed from a checkpoint agree bit for bit.  A vertex force at the
+ * batch, and a run resumed from a checkpoint agree bit for bit (meshes of up to 8192
+ * triangles; larger ones sum their volume by threads per cell).  A vertex force at the
  * limit keeps 49 bits; smaller ones lose relatively more (absolute rounding 2^(e-50)). */
 hc_status hc_set_exact_spread(hc_ctx* ctx, int on);
 hc_status hc_set_repulsion(hc_ctx* ctx, double k_rep, double cutoff_lu, int timescale);
